@@ -592,7 +592,7 @@ def gemm_roofline(step, per, traffic_tab=None, fused=False):
     tops = 2 * step.M * N_ * K_ / (d["avg_us"] * 1e-6) / 1e12
     return dom, {"bound": "mfma", "achieved": round(tops, 2), "peak": INT8_PEAK_TOPS, "unit": "TFLOP/s",
                  "frac": round(tops / INT8_PEAK_TOPS, 4), "traffic": None,
-                 "kernel": f"{dom} GEMM (gemm_pf2_kernel, int8 ops)", "ops_per_launch": 2 * step.M * N_ * K_,
+                 "kernel": f"{dom} GEMM (gemm_t32_kernel, int8 ops)", "ops_per_launch": 2 * step.M * N_ * K_,
                  "avg_launch_us": d["avg_us"]}
 
 

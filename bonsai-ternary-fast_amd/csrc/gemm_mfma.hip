@@ -1,35 +1,22 @@
 // gemm_mfma.hip -- ternary GEMM on T2 codes with int8 MFMA (gfx950), for
-// batched decode and prefill. Same contract as the reference's gemv_kernel
-// (src/cuda/kernels.cu:238-334) for M activation rows. Kernels:
-//   gemm_kp_kernel   up to 16 rows (batched decode): 16 weight rows per
-//                    workgroup, K split over its waves, two 32-column
-//                    sub-blocks of 8 rows per 16x16x64 MFMA, an LDS-direct
-//                    ring per wave;
+// batched decode (up to 32 activation rows; more rows: gemm_t32.hip). Same
+// contract as the reference's gemv_kernel (src/cuda/kernels.cu:238-334).
+// Kernels:
+//   gemm_kp_kernel   up to 16 rows: 16 weight rows per workgroup, K split over
+//                    its waves, two 32-column sub-blocks of 8 rows per
+//                    16x16x64 MFMA, an LDS-direct ring per wave;
 //   gemm_ks_kernel   17 to 32 rows (and up to 16 when d or s are not 16-byte
 //                    aligned): the same workgroup, one sub-block per
-//                    16x16x32 MFMA, staged through registers;
-//   gemm_pf2_kernel  more rows (prefill): 64 weight rows x 64 or 128
-//                    activation rows, fed by an LDS-direct ring;
-//   gemm_pf_kernel   the same tile staged through registers (activation
-//                    scales not 16-byte aligned).
+//                    16x16x32 MFMA, staged through registers.
 // Each has a DUMP instance (btf_hip_gemv_i32_dump) that writes the exact
 // int32 I of every (row, output, sub-block) from the same tile.
 //
-// The prefill tile: a workgroup of 4 waves owns 64 weight rows (swiglu: 32
-// gate rows and the same 32 up rows) and BM = 32 * MW activation rows; the
-// K loop walks 128-column blocks (one fp16 weight scale): codes (64 x 32 B),
-// the block's scales, q (BM x 128 B) and the activation d (BM x 4) are staged
-// in LDS, then every wave runs, per 32-column sub-block,
-//     I = mfma_i32_16x16x32_i8(A = q, B = codes)              (exact int32)
-//     blk += d[m][s] * (float)I
-// and per block acc += fp16(scale[n]) * blk.
 // Lane l of a 16x16x32 MFMA holds A row (l%16) and B column (l%16) bytes for
 // k = 8*(l/16) .. +7; the codes for columns 8t..8t+7 of a sub-block are the
 // 2-bit fields {2(t%2), 2(t%2)+1} of its word t/2, so each lane unpacks its
 // B fragment with two shift+mask ops. C row 4*(l/16)+r, column l%16 lands in
-// accumulator r of lane l. gemm_pf_kernel starts the accumulator at -s (the
-// codes 0 / 1 / 2 as they are); gemm_pf2_kernel and gemm_ks_kernel map the
-// codes to int8 -1 / 0 / +1 (one byte permute per word) and start it at 0.
+// accumulator r of lane l. gemm_ks_kernel maps the codes to int8 -1 / 0 / +1
+// (one byte permute per word) and starts the accumulator at 0.
 #include <climits>
 
 #include "../../include/btf/hip_abi.h"
@@ -69,7 +56,7 @@ struct MfmaArgs {
   int32_t* os;
 };
 
-// ---- LDS-direct loads (the packed K-split tile and the prefill tile) ----
+// ---- LDS-direct loads (the packed K-split tile) ----
 // vmcnt(N) alone (expcnt, lgkmcnt not waited on).
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -103,8 +90,8 @@ __device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
 // staging its own codes, scales, q and d in a private LDS region (the codes
 // are permuted to int8 -1 / 0 / +1, so the MFMA yields I with accumulator 0
 // and s is not read), KB blocks per round. The activation is re-read from L2
-// by each tile. Per wave the row sums follow the prefill tile's order over
-// its blocks (blk = d * I over a block's sub-blocks, acc += scale * blk per
+// by each tile. Per wave the row sums run over its blocks
+// in order (blk = d * I over a block's sub-blocks, acc += scale * blk per
 // block), and the NW wave partials are added in wave order: ((p0 + p1) + p2) + ...
 // TR = 2: the workgroup owns 32 weight rows (two 16-row tiles, each with its
 // gate and up rows), one Q8 block of the output for every activation row, so
@@ -761,486 +748,20 @@ void by_waves_kp(int nw, int mode, const MfmaArgs& a, dim3 grid, hipStream_t st)
     by_mode_kp<4, MG, DUMP, TR>(mode, a, grid, st);
 }
 
-// Prefill tile (more than 32 activation rows): a workgroup owns 64 staged
-// weight rows (swiglu: 32 gate rows and the same 32 up rows) and BM = 32 * MW
-// activation rows; wave (wn, wm) = (w & 1, w >> 1) computes 32 staged rows x
-// 16 * MW activation rows, 2 x MW MFMA tiles per 32-column sub-block from 2 B
-// and MW A fragments (swiglu: its two B tiles are the gate and up rows of the same
-// 16 outputs, so the epilogue stays in the lane). Per output the sums follow
-// this order: blk = d * I over the block's sub-blocks, then
-// acc += scale * blk per block.
-template <int MW, int KB, int MODE, bool DUMP = false>
-__global__ void __launch_bounds__(256) gemm_pf_kernel(MfmaArgs a) {
-  constexpr int BM = 32 * MW;
-  constexpr int CS = 8 * KB + 1;
-  constexpr int QS = 32 * KB + 2;
-  constexpr int NCV = (64 * 2 * KB + 255) / 256;
-  constexpr int NSV = (64 * KB + 255) / 256;
-  constexpr int NQV = (BM * 8 * KB + 255) / 256;
-  constexpr int NDV = (BM * 4 * KB + 255) / 256;
-  constexpr bool SW = MODE == BTF_GEMV_SWIGLU;
-  __shared__ uint32_t cs[64 * CS];
-  __shared__ uint16_t scs[64 * KB];
-  __shared__ uint32_t qsm[BM * QS];
-  __shared__ float dsm[4 * KB][BM];
-  __shared__ int32_t nsm[4 * KB][BM];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = tid >> 6;
-  const int wn = w & 1, wm = w >> 1;
-  const int li = lane & 15;
-  const int t = lane >> 4;
-
-  const int bx = blockIdx.x;
-  const int seg = (bx >= a.tile_start[1]) + (bx >= a.tile_start[2]);
-  const uint8_t* codes = seg == 0 ? a.codes[0] : seg == 1 ? a.codes[1] : a.codes[2];
-  const uint16_t* scales = seg == 0 ? a.scales[0] : seg == 1 ? a.scales[1] : a.scales[2];
-  float* y = seg == 0 ? a.y[0] : seg == 1 ? a.y[1] : a.y[2];
-  const int N = seg == 0 ? a.N[0] : seg == 1 ? a.N[1] : a.N[2];
-  const int ldy = seg == 0 ? a.ldy[0] : seg == 1 ? a.ldy[1] : a.ldy[2];
-  const int tile0 = seg == 0 ? 0 : seg == 1 ? a.tile_start[1] : a.tile_start[2];
-  const int K = a.K;
-  const int rowb = K >> 2, nsc = K >> 7, nsub = a.nsub;
-  constexpr int ROWS_REAL = SW ? 32 : 64;
-  const int n0 = (bx - tile0) * ROWS_REAL;
-  const int mb = blockIdx.y * BM;
-
-  // staged row of this wave's B tile j (lane row li added at use)
-  int srow[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) srow[j] = SW ? 32 * j + 16 * wn : 32 * wn + 16 * j;
-
-  float acc[2][MW][4], blk[2][MW][4];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[j][mt][r] = 0.f;
-
-  u32x4 rc[NCV], rq[NQV];
-  uint16_t rsc[NSV];
-  float rd[NDV];
-  int rs[NDV];
-  auto fetch = [&](int kb0) {
-    const int nkb = nsc - kb0 < KB ? nsc - kb0 : KB;
-#pragma unroll
-    for (int j = 0; j < NCV; ++j) {
-      const int i = tid + 256 * j;
-      const int r = i / (2 * KB), part = i - r * (2 * KB);
-      rc[j] = u32x4{0u, 0u, 0u, 0u};
-      if (i < 64 * 2 * KB && part < 2 * nkb) {
-        const bool up = SW && r >= 32;
-        const int nr = n0 + (SW ? (r & 31) : r);
-        const int nc = nr < N ? nr : N - 1;
-        const uint8_t* cb = up ? a.up_codes : codes;
-        rc[j] = *reinterpret_cast<const u32x4*>(cb + (size_t)nc * rowb + kb0 * 32 + 16 * part);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NSV; ++j) {
-      const int i = tid + 256 * j;
-      const int r = i / KB, jj = i - r * KB;
-      rsc[j] = 0;
-      if (i < 64 * KB && jj < nkb) {
-        const bool up = SW && r >= 32;
-        const int nr = n0 + (SW ? (r & 31) : r);
-        const int nc = nr < N ? nr : N - 1;
-        const uint16_t* sb = up ? a.up_scales : scales;
-        rsc[j] = sb[(size_t)nc * nsc + kb0 + jj];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NQV; ++j) {
-      const int i = tid + 256 * j;
-      const int r = i / (8 * KB), part = i - r * (8 * KB);
-      const int m = mb + r;
-      rq[j] = u32x4{0u, 0u, 0u, 0u};
-      if (i < BM * 8 * KB && part < 8 * nkb && m < a.nb)
-        rq[j] = *reinterpret_cast<const u32x4*>(a.q + (size_t)(a.m0 + m) * K + kb0 * 128 + 16 * part);
-    }
-#pragma unroll
-    for (int j = 0; j < NDV; ++j) {
-      const int i = tid + 256 * j;
-      const int r = i / (4 * KB), sb = i - r * (4 * KB);
-      const int m = mb + r;
-      rd[j] = 0.f;
-      rs[j] = 0;
-      if (i < BM * 4 * KB && sb < 4 * nkb && m < a.nb) {
-        const size_t o = (size_t)(a.m0 + m) * nsub + kb0 * 4 + sb;
-        rd[j] = a.d[o];
-        rs[j] = a.s[o];
-      }
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int j = 0; j < NCV; ++j) {
-      const int i = tid + 256 * j;
-      if (i < 64 * 2 * KB) {
-        const int r = i / (2 * KB), part = i - r * (2 * KB);
-        uint32_t* o = &cs[r * CS + 4 * part];
-        o[0] = rc[j].x; o[1] = rc[j].y; o[2] = rc[j].z; o[3] = rc[j].w;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NSV; ++j) {
-      const int i = tid + 256 * j;
-      if (i < 64 * KB) scs[i] = rsc[j];
-    }
-#pragma unroll
-    for (int j = 0; j < NQV; ++j) {
-      const int i = tid + 256 * j;
-      if (i < BM * 8 * KB) {
-        const int r = i / (8 * KB), part = i - r * (8 * KB);
-        uint32_t* o = &qsm[r * QS + 4 * part];
-        o[0] = rq[j].x; o[1] = rq[j].y; o[2] = rq[j].z; o[3] = rq[j].w;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NDV; ++j) {
-      const int i = tid + 256 * j;
-      if (i < BM * 4 * KB) {
-        const int r = i / (4 * KB), sb = i - r * (4 * KB);
-        dsm[sb][r] = rd[j];
-        nsm[sb][r] = -rs[j];
-      }
-    }
-  };
-
-  fetch(0);
-  for (int kb0 = 0; kb0 < nsc; kb0 += KB) {
-    const int nkb = nsc - kb0 < KB ? nsc - kb0 : KB;
-    stage();
-    __syncthreads();
-    if (kb0 + KB < nsc) fetch(kb0 + KB);  // in flight while this stage is dotted
-
-    for (int kbi = 0; kbi < nkb; ++kbi) {
-#pragma unroll
-      for (int sb = 0; sb < 4; ++sb) {
-        const int sbx = 4 * kbi + sb;
-        long bfrag[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint32_t word = cs[(srow[j] + li) * CS + 2 * sbx + (t >> 1)];
-          const int sh = 4 * (t & 1);
-          const uint32_t lo = (word >> sh) & 0x03030303u;
-          const uint32_t hi = (word >> (sh + 2)) & 0x03030303u;
-          bfrag[j] = (long)(((uint64_t)hi << 32) | lo);
-        }
-#pragma unroll
-        for (int mt = 0; mt < MW; ++mt) {
-          const int mr = 16 * MW * wm + 16 * mt;
-          const uint32_t* ap = &qsm[(mr + li) * QS + 8 * sbx + 2 * t];
-          const long afrag = (long)(((uint64_t)ap[1] << 32) | ap[0]);
-          v4i cin;
-          float dv[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            cin[r] = nsm[sbx][mr + 4 * t + r];
-            dv[r] = dsm[sbx][mr + 4 * t + r];
-          }
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const v4i I = __builtin_amdgcn_mfma_i32_16x16x32_i8(afrag, bfrag[j], cin, 0, 0, 0);
-            if constexpr (DUMP) {  // the exact I of every (row, output, sub-block), as launched
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const int m = mb + mr + 4 * t + r, n = n0 + srow[j] + li;
-                if (m < a.nb && n < N) a.dump[((size_t)(a.m0 + m) * N + n) * nsub + (kb0 + kbi) * 4 + sb] = I[r];
-              }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              blk[j][mt][r] = sb == 0 ? dv[r] * (float)I[r] : fmaf(dv[r], (float)I[r], blk[j][mt][r]);
-          }
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float sc = h2f(scs[(srow[j] + li) * KB + kbi]);
-#pragma unroll
-        for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[j][mt][r] = fmaf(sc, blk[j][mt][r], acc[j][mt][r]);
-      }
-    }
-    __syncthreads();
-  }
-  if constexpr (DUMP) return;
-
-#pragma unroll
-  for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = mb + 16 * MW * wm + 16 * mt + 4 * t + r;
-      if (m >= a.nb) continue;
-      if constexpr (SW) {
-        const int n = n0 + 16 * wn + li;
-        if (n < N) {
-          const float g = acc[0][mt][r], u = acc[1][mt][r];
-          y[(size_t)(a.m0 + m) * ldy + n] = g / (1.0f + expf(-g)) * u;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int n = n0 + srow[j] + li;
-          if (n < N) {
-            float* o = &y[(size_t)(a.m0 + m) * ldy + n];
-            if constexpr (MODE == BTF_GEMV_ADD)
-              *o += acc[j][mt][r];
-            else
-              *o = acc[j][mt][r];
-          }
-        }
-      }
-    }
-}
-
-template <int MW>
-void by_mode_pf(int mode, const MfmaArgs& a, dim3 grid, hipStream_t st) {
-  constexpr int KB = 1;
-  if (mode == BTF_GEMV_STORE)
-    hipLaunchKernelGGL((gemm_pf_kernel<MW, KB, BTF_GEMV_STORE>), grid, dim3(256), 0, st, a);
-  else if (mode == BTF_GEMV_ADD)
-    hipLaunchKernelGGL((gemm_pf_kernel<MW, KB, BTF_GEMV_ADD>), grid, dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((gemm_pf_kernel<MW, KB, BTF_GEMV_SWIGLU>), grid, dim3(256), 0, st, a);
-}
-
-// The prefill tile of gemm_pf_kernel (64 staged weight rows x BM = 32 * MW
-// activation rows, wave (w & 1, w >> 1) computes 32 x 16 * MW) fed by an
-// S-stage ring of LDS-direct loads: after the barrier of block k each wave
-// issues its share of block k + S - 1, so a load has S - 1 blocks of compute
-// to arrive in and no staging registers. The 2-bit codes are mapped to int8
-// {-1, 0, +1} with one byte permute per word, so the MFMA yields
-// I = sum q * w directly (accumulator 0) and s is not read. Stage layout:
-// q [BM][128 B] with the 16-byte chunk c of row r at slot c ^ (r & 7) (the A
-// fragments of 16 rows fall in 8 bank groups), codes [64][2 x 16 B] with the
-// halves of row r swapped when bit 3 of r is set (rows r and r + 8 of a
-// fragment read then fall in different banks), d [BM][4], scales [64] in
-// 4-byte slots. Same sums, in the same order, as gemm_pf_kernel.
-template <int MW, int S, int MODE, bool DUMP = false>
-__global__ void __launch_bounds__(256) gemm_pf2_kernel(MfmaArgs a) {
-  constexpr int BM = 32 * MW;
-  constexpr bool SW = MODE == BTF_GEMV_SWIGLU;
-  constexpr int QB = BM * 128, CB = 64 * 32, DB = BM * 16, SCB = 64 * 4;
-  constexpr int STG = QB + CB + DB + SCB;
-  constexpr int NQ = BM / 32;  // q loads per wave per block
-  static_assert(STG % 16 == 0, "stage alignment");
-  __shared__ __attribute__((aligned(16))) uint8_t ring[S * STG];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: LDS bases and roles
-  const int wn = w & 1, wm = w >> 1;
-  const int li = lane & 15;
-  const int t = lane >> 4;
-
-  const int bx = blockIdx.x;
-  const int seg = (bx >= a.tile_start[1]) + (bx >= a.tile_start[2]);
-  const uint8_t* codes = seg == 0 ? a.codes[0] : seg == 1 ? a.codes[1] : a.codes[2];
-  const uint16_t* scales = seg == 0 ? a.scales[0] : seg == 1 ? a.scales[1] : a.scales[2];
-  float* y = seg == 0 ? a.y[0] : seg == 1 ? a.y[1] : a.y[2];
-  const int N = seg == 0 ? a.N[0] : seg == 1 ? a.N[1] : a.N[2];
-  const int ldy = seg == 0 ? a.ldy[0] : seg == 1 ? a.ldy[1] : a.ldy[2];
-  const int tile0 = seg == 0 ? 0 : seg == 1 ? a.tile_start[1] : a.tile_start[2];
-  const int K = a.K;
-  const int rowb = K >> 2, nsc = K >> 7, nsub = a.nsub;
-  constexpr int ROWS_REAL = SW ? 32 : 64;
-  const int n0 = (bx - tile0) * ROWS_REAL;
-  const int mb = blockIdx.y * BM;
-  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;  // LDS byte address
-
-  // ---- this lane's load sources (block 0; block kb adds kb * step) ----
-  // q: load i covers slots (w * NQ + i) * 64 + lane -> row P / 8, slot P % 8
-  const int8_t* qsrc[NQ];
-#pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    const int P = (w * NQ + i) * 64 + lane;
-    const int r = P >> 3, c = (P & 7) ^ (r & 7);
-    const int m = mb + r < a.nb ? mb + r : a.nb - 1;
-    qsrc[i] = a.q + (size_t)(a.m0 + m) * K + 16 * c;
-  }
-  // codes (waves 0, 1): slot P = w * 64 + lane -> staged row P / 2, slot P % 2
-  // holding half (P % 2) ^ (bit 3 of the row)
-  const uint8_t* csrc;
-  {
-    const int P = (w & 1) * 64 + lane;
-    const int r = P >> 1;
-    const int nr = n0 + (SW ? (r & 31) : r);
-    const int nc = nr < N ? nr : N - 1;
-    csrc = (SW && r >= 32 ? a.up_codes : codes) + (size_t)nc * rowb + 16 * ((P & 1) ^ ((r >> 3) & 1));
-  }
-  // d (waves 2, 3): row (w - 2) * 64 + lane; scales (wave 3): staged row lane
-  const float* dsrc;
-  {
-    const int r = ((w - 2) & 1) * 64 + lane;
-    const int m = mb + r < a.nb ? mb + r : a.nb - 1;
-    dsrc = a.d + (size_t)(a.m0 + m) * nsub;
-  }
-  const uint16_t* ssrc;
-  {
-    const int nr = n0 + (SW ? (lane & 31) : lane);
-    const int nc = nr < N ? nr : N - 1;
-    ssrc = (SW && lane >= 32 ? a.up_scales : scales) + (size_t)nc * nsc;
-  }
-  // Loads per wave per block: NQ q + (waves 0, 1: codes; waves 2, 3: d when
-  // BM covers them) + (wave 3: scales).
-  const bool do_d = w >= 2 && (w - 2) * 64 < BM;
-  auto issue = [&](int kb) {
-    const int kc = kb < nsc ? kb : nsc - 1;  // blocks past the end reload the last (never read)
-    const uint32_t st = ring0 + (uint32_t)((kb % S) * STG);
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) lds_dma16(qsrc[i] + (size_t)kc * 128, st + (uint32_t)((w * NQ + i) * 1024));
-    if (w < 2) lds_dma16(csrc + (size_t)kc * 32, st + QB + (uint32_t)(w * 1024));
-    if (do_d) lds_dma16(dsrc + (size_t)kc * 4, st + QB + CB + (uint32_t)((w - 2) * 1024));
-    if (w == 3) lds_dma2(ssrc + kc, st + QB + CB + DB);
-  };
-
-  int srow[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) srow[j] = SW ? 32 * j + 16 * wn : 32 * wn + 16 * j;
-
-  float acc[2][MW][4], blk[2][MW][4];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[j][mt][r] = 0.f;
-
-#pragma unroll
-  for (int kb = 0; kb < S - 1; ++kb) issue(kb);
-  const v4i zero = {0, 0, 0, 0};
-  for (int kb = 0; kb < nsc; ++kb) {
-    // this wave's loads of block kb have landed once at most (S - 2) blocks of
-    // its loads are outstanding
-    constexpr int L012 = NQ + 1, L3 = NQ + (BM > 64 ? 1 : 0) + 1;
-    if (w == 3)
-      wait_vm<L3 * (S - 2)>();
-    else
-      wait_vm<L012 * (S - 2)>();
-    __syncthreads();  // every wave's loads of kb landed; every wave is done with block kb - 1
-    issue(kb + S - 1);  // into the stage of block kb - 1
-    const uint8_t* stg = ring + (kb % S) * STG;
-    const uint8_t* cst = stg + QB;
-    const float* dst = reinterpret_cast<const float*>(stg + QB + CB);
-    const uint8_t* sst = stg + QB + CB + DB;
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb) {
-      long bfrag[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int wi = 2 * sb + (t >> 1);  // word of the staged row (half wi / 4, stored swapped for rows 8-15 of 16)
-        const uint32_t word =
-            *reinterpret_cast<const uint32_t*>(cst + (srow[j] + li) * 32 + 16 * ((wi >> 2) ^ (li >> 3)) + 4 * (wi & 3));
-        const int sh = 4 * (t & 1);
-        const uint32_t lo = __builtin_amdgcn_perm(0u, 0x000100FFu, (word >> sh) & 0x03030303u);
-        const uint32_t hi = __builtin_amdgcn_perm(0u, 0x000100FFu, (word >> (sh + 2)) & 0x03030303u);
-        bfrag[j] = (long)(((uint64_t)hi << 32) | lo);
-      }
-      // every MFMA of the sub-block first, into its own registers, then the
-      // scaling: the matrix core runs the next products while the vector ALU
-      // converts the earlier ones (one result register set, reused, would
-      // make each MFMA wait for the conversions of the one before)
-      v4i I[MW][2];
-#pragma unroll
-      for (int mt = 0; mt < MW; ++mt) {
-        const int r = 16 * MW * wm + 16 * mt + li;
-        const long afrag = *reinterpret_cast<const long*>(stg + r * 128 + 16 * ((2 * sb + (t >> 1)) ^ (r & 7)) +
-                                                          8 * (t & 1));
-#pragma unroll
-        for (int j = 0; j < 2; ++j) I[mt][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(afrag, bfrag[j], zero, 0, 0, 0);
-      }
-      if constexpr (DUMP) {  // the exact I of every (row, output, sub-block), as launched
-#pragma unroll
-        for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-              const int m = mb + 16 * MW * wm + 16 * mt + 4 * t + rr, n = n0 + srow[j] + li;
-              if (m < a.nb && n < N) a.dump[((size_t)(a.m0 + m) * N + n) * nsub + kb * 4 + sb] = I[mt][j][rr];
-            }
-      }
-#pragma unroll
-      for (int mt = 0; mt < MW; ++mt) {
-        const int mr = 16 * MW * wm + 16 * mt;
-        float dv[4];
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) dv[rr] = dst[(mr + 4 * t + rr) * 4 + sb];
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr)
-            blk[j][mt][rr] =
-                sb == 0 ? dv[rr] * (float)I[mt][j][rr] : fmaf(dv[rr], (float)I[mt][j][rr], blk[j][mt][rr]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float sc = h2f(*reinterpret_cast<const uint16_t*>(sst + 4 * (srow[j] + li)));
-#pragma unroll
-      for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[j][mt][r] = fmaf(sc, blk[j][mt][r], acc[j][mt][r]);
-    }
-  }
-  wait_vm<0>();  // the trailing loads land before the workgroup's LDS is released
-  if constexpr (DUMP) return;
-
-#pragma unroll
-  for (int mt = 0; mt < MW; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = mb + 16 * MW * wm + 16 * mt + 4 * t + r;
-      if (m >= a.nb) continue;
-      if constexpr (SW) {
-        const int n = n0 + 16 * wn + li;
-        if (n < N) {
-          const float g = acc[0][mt][r], u = acc[1][mt][r];
-          y[(size_t)(a.m0 + m) * ldy + n] = g / (1.0f + expf(-g)) * u;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int n = n0 + srow[j] + li;
-          if (n < N) {
-            float* o = &y[(size_t)(a.m0 + m) * ldy + n];
-            if constexpr (MODE == BTF_GEMV_ADD)
-              *o += acc[j][mt][r];
-            else
-              *o = acc[j][mt][r];
-          }
-        }
-      }
-    }
-}
-
-template <int MW, int S>
-void by_mode_pf2(int mode, const MfmaArgs& a, dim3 grid, hipStream_t st) {
-  if (mode == BTF_GEMV_STORE)
-    hipLaunchKernelGGL((gemm_pf2_kernel<MW, S, BTF_GEMV_STORE>), grid, dim3(256), 0, st, a);
-  else if (mode == BTF_GEMV_ADD)
-    hipLaunchKernelGGL((gemm_pf2_kernel<MW, S, BTF_GEMV_ADD>), grid, dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((gemm_pf2_kernel<MW, S, BTF_GEMV_SWIGLU>), grid, dim3(256), 0, st, a);
-}
-
 }  // namespace
 
 int mfma_rows_per_pass() { return 64; }
 
 int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-              hipStream_t st, const DevState& ds, const Q8* qout) {
+              hipStream_t st, const DevState&, const Q8* qout) {
   MfmaArgs a{};
-  // up to 32 activation rows: the K-split 16-row tile (32 rows with a Q8
-  // output); more: the prefill tile
-  const bool ks = nb <= 32;
-  if (qout && (!ks || dump)) return fail(BTF_ERR_ARGS, "gemm: a Q8 output needs at most 32 rows");
-  const int rows_real = ks ? (qout ? 32 : 16) : mode == BTF_GEMV_SWIGLU ? 32 : 64;
+  if (nb > 32) {
+    if (qout) return fail(BTF_ERR_ARGS, "gemm: a Q8 output needs at most 32 rows");
+    return gemm_t32(segs, nseg, K, m0, nb, act, mode, dump, st);
+  }
+  // the K-split 16-row tile (32 rows with a Q8 output)
+  if (qout && dump) return fail(BTF_ERR_ARGS, "gemm: a Q8 output has no dump");
+  const int rows_real = qout ? 32 : 16;
   const int nuse = mode == BTF_GEMV_SWIGLU ? 1 : nseg;
   int tiles = 0;
   for (int i = 0; i < 3; ++i) {
@@ -1274,75 +795,44 @@ int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& ac
     a.os = const_cast<int32_t*>(qout->s);
   }
   if (tiles == 0) return BTF_OK;
-  const int MT = nb <= 16 ? 1 : nb <= 32 ? 2 : 4;
+  const int MT = nb <= 16 ? 1 : 2;
   const int BM = 16 * MT;
   const dim3 grid(tiles, (nb + BM - 1) / BM);
   const bool dmp = dump != nullptr;
-  if (ks) {
-    // up to 16 rows with d and s 16-byte aligned (the LDS-direct loads of the
-    // packed tile read them in 16-byte pieces): the packed tile
-    const int kw = kp_waves(K, mode);
-    if (nb <= 16 && kw && ((reinterpret_cast<uintptr_t>(act.d) | reinterpret_cast<uintptr_t>(act.s)) & 15) == 0) {
-      const dim3 gk(tiles, 1);
-      if (qout) {
-        if (nb <= 8)
-          by_waves_kp<1, false, 2>(kw, mode, a, gk, st);
-        else
-          by_waves_kp<2, false, 2>(kw, mode, a, gk, st);
-      } else if (nb <= 8) {
-        dmp ? by_waves_kp<1, true>(kw, mode, a, gk, st) : by_waves_kp<1, false>(kw, mode, a, gk, st);
-      } else {
-        dmp ? by_waves_kp<2, true>(kw, mode, a, gk, st) : by_waves_kp<2, false>(kw, mode, a, gk, st);
-      }
-      return launch_status("gemm_kp_kernel");
-    }
-    // 8 waves split K for one activation tile (measured: down 29.6 -> 25.2 us and
-    // QKV 11.0 -> 10.1 us at M = 8), except gate+up at K = 5120 (27 -> 31 us);
-    // with two activation tiles 8 waves were slower on every shape
-    const int nw = MT == 1 && (K >= 8192 || mode != BTF_GEMV_SWIGLU) ? 8 : 4;
-    // (the K split depends on nw only: the outputs do not depend on the tile height)
+  // up to 16 rows with d and s 16-byte aligned (the LDS-direct loads of the
+  // packed tile read them in 16-byte pieces): the packed tile
+  const int kw = kp_waves(K, mode);
+  if (nb <= 16 && kw && ((reinterpret_cast<uintptr_t>(act.d) | reinterpret_cast<uintptr_t>(act.s)) & 15) == 0) {
+    const dim3 gk(tiles, 1);
     if (qout) {
-      if (MT == 1)
-        by_waves_ks<1, false, 2>(nw, mode, a, grid, st);
+      if (nb <= 8)
+        by_waves_kp<1, false, 2>(kw, mode, a, gk, st);
       else
-        by_waves_ks<2, false, 2>(nw, mode, a, grid, st);
-      return launch_status("gemm_ks_kernel");
+        by_waves_kp<2, false, 2>(kw, mode, a, gk, st);
+    } else if (nb <= 8) {
+      dmp ? by_waves_kp<1, true>(kw, mode, a, gk, st) : by_waves_kp<1, false>(kw, mode, a, gk, st);
+    } else {
+      dmp ? by_waves_kp<2, true>(kw, mode, a, gk, st) : by_waves_kp<2, false>(kw, mode, a, gk, st);
     }
+    return launch_status("gemm_kp_kernel");
+  }
+  // 8 waves split K for one activation tile (measured: down 29.6 -> 25.2 us and
+  // QKV 11.0 -> 10.1 us at M = 8), except gate+up at K = 5120 (27 -> 31 us);
+  // with two activation tiles 8 waves were slower on every shape
+  const int nw = MT == 1 && (K >= 8192 || mode != BTF_GEMV_SWIGLU) ? 8 : 4;
+  // (the K split depends on nw only: the outputs do not depend on the tile height)
+  if (qout) {
     if (MT == 1)
-      dmp ? by_waves_ks<1, true>(nw, mode, a, grid, st) : by_waves_ks<1, false>(nw, mode, a, grid, st);
+      by_waves_ks<1, false, 2>(nw, mode, a, grid, st);
     else
-      dmp ? by_waves_ks<2, true>(nw, mode, a, grid, st) : by_waves_ks<2, false>(nw, mode, a, grid, st);
+      by_waves_ks<2, false, 2>(nw, mode, a, grid, st);
     return launch_status("gemm_ks_kernel");
   }
-  // 128 activation rows per tile while that still gives two workgroups per CU, else 64
-  const int cus = ds.cu_count > 0 ? ds.cu_count : 256;
-  const bool wide = (int64_t)tiles * ((nb + 127) / 128) >= 2 * cus;
-  const dim3 gw(tiles, (nb + 127) / 128), gn(tiles, (nb + 63) / 64);
-  // the LDS-direct ring loads d in 16-byte pieces
-  if ((reinterpret_cast<uintptr_t>(act.d) & 15) == 0) {
-    if (dmp) {  // the exact-I dump (btf_hip_gemv_i32_dump, one matrix): the same tile, writing I
-      if (wide)
-        hipLaunchKernelGGL((gemm_pf2_kernel<4, 2, BTF_GEMV_STORE, true>), gw, dim3(256), 0, st, a);
-      else
-        hipLaunchKernelGGL((gemm_pf2_kernel<2, 3, BTF_GEMV_STORE, true>), gn, dim3(256), 0, st, a);
-    } else if (wide) {
-      by_mode_pf2<4, 2>(mode, a, gw, st);  // 41 KB; 190 VGPRs: 2 workgroups per CU
-    } else {
-      by_mode_pf2<2, 3>(mode, a, gn, st);  // 34 KB: 4 workgroups per CU
-    }
-    return launch_status("gemm_pf2_kernel");
-  }
-  if (dmp) {
-    if (wide)
-      hipLaunchKernelGGL((gemm_pf_kernel<4, 1, BTF_GEMV_STORE, true>), gw, dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((gemm_pf_kernel<2, 1, BTF_GEMV_STORE, true>), gn, dim3(256), 0, st, a);
-  } else if (wide) {
-    by_mode_pf<4>(mode, a, gw, st);
-  } else {
-    by_mode_pf<2>(mode, a, gn, st);
-  }
-  return launch_status("gemm_pf_kernel");
+  if (MT == 1)
+    dmp ? by_waves_ks<1, true>(nw, mode, a, grid, st) : by_waves_ks<1, false>(nw, mode, a, grid, st);
+  else
+    dmp ? by_waves_ks<2, true>(nw, mode, a, grid, st) : by_waves_ks<2, false>(nw, mode, a, grid, st);
+  return launch_status("gemm_ks_kernel");
 }
 
 }  // namespace btfhip

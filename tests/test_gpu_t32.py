@@ -1,0 +1,116 @@
+"""The 32x32-tile GEMM (more than 32 activation rows) in each of its four tile
+shapes, at the edges of tiles, segments and K groups.
+
+Oracle: the exact int32 I of the oracle, scaled and summed in float64. An
+output is one rounding per sub-block product, at most four per 128-column
+block inside it, one per block of a group's chain and one per group, so
+    |y - y64| <= (nblocks + 16) * 2^-24 * sum |scale * d * I|
+(each rounding is at most 2^-24 of a partial sum that the sum of magnitudes
+bounds); swiglu adds its own few roundings (2^-20 of the product's bound,
+expf within 2 ulp, and the derivative of silu below 1.1).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _torch():
+    import torch
+    return torch
+
+
+def dev(a):
+    torch = _torch()
+    a = np.ascontiguousarray(a)
+    if a.dtype == np.uint16:
+        a = a.view(np.int16)
+    return torch.from_numpy(a.copy()).cuda()
+
+
+def stream():
+    return _torch().cuda.current_stream().cuda_stream
+
+
+def matrix(rng, N, K):
+    """Codes with P(-1, 0, +1) = (0.3, 0.4, 0.3) and scales in [0.01, 0.05]."""
+    c = rng.choice(3, p=[0.3, 0.4, 0.3], size=(4096, 4)).astype(np.uint8)
+    lut = c[:, 0] | c[:, 1] << 2 | c[:, 2] << 4 | c[:, 3] << 6
+    codes = lut[rng.integers(0, 4096, (N, K // 4))]
+    scales = (0.01 + 0.04 * rng.random((N, K // 128))).astype(np.float16).view(np.uint16)
+    return codes, scales
+
+
+def wide(oracle, mat, sel, K, q, d, s):
+    """(y, sum of magnitudes) of the sampled rows in float64, [M][len(sel)]."""
+    codes, scales = np.ascontiguousarray(mat[0][sel]), mat[1][sel].view(np.float16).astype(np.float64)
+    I = oracle.gemv_i32(codes, K, q, s).astype(np.float64)
+    t = I * d.astype(np.float64)[:, None, :] * np.repeat(scales, 4, axis=1)[None]
+    return t.sum(-1), np.abs(t).sum(-1)
+
+
+# (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses
+CASES = [
+    (128, 33, [1, 33], 1),           # one block: seven of eight K groups have none
+    (384, 64, [37, 70, 9], 17),      # three blocks over eight groups, three segments
+    (1152, 95, [45], 50),            # nine blocks: uneven groups, a dead row in the last tile
+    (640, 65, [6917], 3500),         # 651 / 657 tiles: two waves x four groups; five blocks
+    (256, 200, [18733], 9400),       # 4102 / 4116 tiles: four waves, K unsplit
+    (256, 513, [15500], 7800),       # 8245 / 8296 tiles: 64 activation rows a wave, the last tile nearly empty
+]
+
+
+@pytest.mark.parametrize("K,M,Ns,N2", CASES)
+def test_t32_modes_and_edges(hip, oracle, K, M, Ns, N2):
+    torch = _torch()
+    G = hip.GemvMode
+    rng = np.random.default_rng(K + M)
+    x = (rng.standard_normal((M, K)) * np.exp(rng.standard_normal((M, 1)))).astype(np.float32)
+    q, d, s = oracle.quantize_rows(x)
+    act = hip.Q8Act(dev(q), dev(d), dev(s))
+    nblk = K // 128
+
+    def check(got, want, mag, what):
+        bound = (nblk + 16) * 2.0 ** -24 * mag
+        bad = np.argwhere(np.abs(got.astype(np.float64) - want) > bound)
+        assert bad.size == 0, f"{what}: {len(bad)} outputs past the bound, first {bad[0]}"
+
+    def sample(N):
+        return np.unique(np.r_[0:min(N, 40), max(0, N // 2 - 20):N // 2, max(0, N - 40):N])
+
+    mats = [matrix(rng, n, K) for n in Ns]
+    ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in Ns]
+    segs = [hip.GemvSeg(dev(c), dev(sc), n, y, n + 3) for (c, sc), n, y in zip(mats, Ns, ys)]
+    hip.launch_gemv(segs, K, M, act, G.kStore, stream())
+    for mat, n, y in zip(mats, Ns, ys):
+        sel = sample(n)
+        want, mag = wide(oracle, mat, sel, K, q, d, s)
+        got = y.cpu().numpy()
+        check(got[:, sel], want, mag, f"store N={n}")
+        assert np.all(got[:, n:] == 7.0), "wrote past N"
+
+    y0 = rng.standard_normal((M, Ns[0])).astype(np.float32)
+    y = dev(y0)
+    hip.launch_gemv([hip.GemvSeg(segs[0].codes, segs[0].scales, Ns[0], y, Ns[0])], K, M, act, G.kAdd, stream())
+    sel = sample(Ns[0])
+    want, mag = wide(oracle, mats[0], sel, K, q, d, s)
+    check(y.cpu().numpy()[:, sel], want + y0[:, sel], mag + np.abs(y0[:, sel]), "add")
+
+    gate, up = matrix(rng, N2, K), matrix(rng, N2, K)
+    y = torch.full((M, N2 + 1), 7.0, device="cuda")
+    hip.launch_gemv([hip.GemvSeg(dev(gate[0]), dev(gate[1]), N2, y, N2 + 1),
+                     hip.GemvSeg(dev(up[0]), dev(up[1]), N2, None, 0)], K, M, act, G.kSwiglu, stream())
+    sel = sample(N2)
+    g, gm = wide(oracle, gate, sel, K, q, d, s)
+    u, um = wide(oracle, up, sel, K, q, d, s)
+    silu = g / (1 + np.exp(-g))
+    got = y.cpu().numpy()
+    bound = (nblk + 16) * 2.0 ** -24 * (1.1 * gm * np.abs(u) + np.abs(silu) * um) * 1.01 + 2.0 ** -20 * np.abs(silu * u)
+    bad = np.argwhere(np.abs(got[:, sel] - silu * u) > bound)
+    assert bad.size == 0, f"swiglu: {len(bad)} outputs past the bound, first {bad[0]}"
+    assert np.all(got[:, N2:] == 7.0), "wrote past N"
+
+    n = min(Ns[-1], 70)  # I of the exact dump, the tile chosen as for a launch of that size
+    I = torch.full((M, n, K // 32), -(1 << 30), dtype=torch.int32, device="cuda")
+    hip.gemv_i32_dump(dev(mats[-1][0][:n]), n, K, M, act, I, stream())
+    assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(np.ascontiguousarray(mats[-1][0][:n]), K, q, s))
