@@ -65,8 +65,9 @@ __device__ __forceinline__ void pair32(float v, float& lo, float& hi) {
 //    every pair of both entries, and swapping those two back puts each
 //    entry's sums in its lower lanes and differences in its upper lanes: two
 //    swaps, an add and a subtract per two entries.
-template <int X>
-__device__ __forceinline__ void xstage(float (&v)[16], int lane) {
+template <int X, int NV>
+__device__ __forceinline__ void xstage(float (&v)[NV], int lane) {
+  static_assert(NV % 4 == 0, "four values at a time");
   // Four values (two pairs) at a time: each value a DPP or permlane
   // instruction reads is written two or more instructions before it, so no
   // wait states go between them (one value at a time, the compiler reused one
@@ -78,7 +79,7 @@ __device__ __forceinline__ void xstage(float (&v)[16], int lane) {
     constexpr int kBit = X == 1 ? 0 : X == 2 ? 1 : X == 4 ? 2 : 3;
     const uint32_t flip = ((uint32_t)lane >> kBit & 1u) << 31;  // the upper lane negates its own value
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
+    for (int i = 0; i < NV; i += 4) {
       float t[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) t[k] = __uint_as_float(__float_as_uint(v[i + k]) ^ flip);
@@ -102,7 +103,7 @@ __device__ __forceinline__ void xstage(float (&v)[16], int lane) {
       hi = __uint_as_float(r[1]);
     };
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
+    for (int i = 0; i < NV; i += 4) {
       float lo[2], hi[2], sm[2], df[2];
 #pragma unroll
       for (int k = 0; k < 2; ++k) swap(v[i + 2 * k], v[i + 2 * k + 1], lo[k], hi[k]);
@@ -121,10 +122,10 @@ __device__ __forceinline__ void xstage(float (&v)[16], int lane) {
 // `block`-sized run of consecutive values (block a power of two, 1..1024;
 // block <= 1 is no transform). Uniform control flow: `block` is the same in
 // every lane.
-template <int LEN>
-__device__ __forceinline__ void istage(float (&v)[16]) {  // an in-lane stage
+template <int LEN, int NV>
+__device__ __forceinline__ void istage(float (&v)[NV]) {  // an in-lane stage
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int j = 0; j < NV; ++j) {
     if (j & LEN) continue;
     const float a = v[j], b = v[j + LEN];
     v[j] = a + b;
@@ -249,29 +250,6 @@ __device__ __forceinline__ double pair_sumsq(const float (&v)[16]) {
   t[1] = t[2] + t[3];
   t[0] = t[0] + t[1];
   return t[0] + lane_xor_d<1>(t[0]);
-}
-
-// The same canonical sum of squares of a 32-value block held in one lane
-// (lo = values 0..15, hi = values 16..31).
-__device__ __forceinline__ double block_sumsq(const float (&lo)[16], const float (&hi)[16]) {
-  double t[16];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const double a = (double)lo[2 * i], b = (double)lo[2 * i + 1];
-    const double c = (double)hi[2 * i], d = (double)hi[2 * i + 1];
-    const double sa = a * a, sb = b * b, sc = c * c, sd = d * d;
-    t[i] = sa + sb;
-    t[8 + i] = sc + sd;
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t[8 * h + i] = t[8 * h + 2 * i] + t[8 * h + 2 * i + 1];
-    t[8 * h] = t[8 * h] + t[8 * h + 1];
-    t[8 * h + 1] = t[8 * h + 2] + t[8 * h + 3];
-    t[8 * h] = t[8 * h] + t[8 * h + 1];
-  }
-  return t[0] + t[8];
 }
 
 // Sum over the wave of one double per lane, every lane getting the total:
