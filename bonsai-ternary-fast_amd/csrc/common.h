@@ -168,9 +168,9 @@ int gemv_b3(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& a, i
 // qout: also the Q8 of the output rows (nb <= 32, N % 32 == 0), for the next GEMM.
 int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& a, int mode, int32_t* dump,
               hipStream_t st, const DevState& ds, const Q8* qout = nullptr);
-// 32x32-tile MFMA path (more than 32 rows).
+// 32x32-tile MFMA path (more than 16 rows). qout: also the Q8 of the output rows (nb <= 32, N % 32 == 0).
 int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-             hipStream_t st);
+             hipStream_t st, const Q8* qout = nullptr);
 int mfma_rows_per_pass();
 
 int repack(const uint8_t* src, int64_t nblocks, uint8_t* codes, uint16_t* scales, hipStream_t st,

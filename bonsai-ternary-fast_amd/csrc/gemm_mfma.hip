@@ -1,13 +1,13 @@
 // gemm_mfma.hip -- ternary GEMM on T2 codes with int8 MFMA (gfx950), for
-// batched decode (up to 32 activation rows; more rows: gemm_t32.hip). Same
+// batched decode (up to 16 activation rows; more rows: gemm_t32.hip). Same
 // contract as the reference's gemv_kernel (src/cuda/kernels.cu:238-334).
 // Kernels:
-//   gemm_kp_kernel   up to 16 rows: 16 weight rows per workgroup, K split over
-//                    its waves, two 32-column sub-blocks of 8 rows per
-//                    16x16x64 MFMA, an LDS-direct ring per wave;
-//   gemm_ks_kernel   17 to 32 rows (and up to 16 when d or s are not 16-byte
-//                    aligned): the same workgroup, one sub-block per
-//                    16x16x32 MFMA, staged through registers.
+//   gemm_kp_kernel   16 weight rows per workgroup, K split over its waves, two
+//                    32-column sub-blocks of 8 rows per 16x16x64 MFMA, an
+//                    LDS-direct ring per wave;
+//   gemm_ks_kernel   the same workgroup, one sub-block per 16x16x32 MFMA,
+//                    staged through registers: where d or s are not 16-byte
+//                    aligned or K is longer than the packed tile takes.
 // Each has a DUMP instance (btf_hip_gemv_i32_dump) that writes the exact
 // int32 I of every (row, output, sub-block) from the same tile.
 //
@@ -84,7 +84,7 @@ __device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
                : "memory");
 }
 
-// K-split tile for batched decode (up to 32 activation rows): a workgroup of
+// K-split tile for batched decode (up to 16 activation rows): a workgroup of
 // NW waves owns 16 weight rows (swiglu: 16 gate rows and the same 16 up rows)
 // and BM activation rows, and wave w walks its 1/NW of the 128-column blocks,
 // staging its own codes, scales, q and d in a private LDS region (the codes
@@ -97,8 +97,9 @@ __device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
 // gate and up rows), one Q8 block of the output for every activation row, so
 // it also writes the Q8 of its outputs (a.oq) with the q8 kernel's
 // arithmetic. The per-output sums do not depend on TR.
-template <int NW, int MT, int KB, int MODE, bool DUMP, int TR = 1>
+template <int NW, int KB, int MODE, bool DUMP, int TR = 1>
 __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
+  constexpr int MT = 1;  // 16-row activation tiles
   constexpr int BM = 16 * MT;
   constexpr int G1 = MODE == BTF_GEMV_SWIGLU ? 2 : 1;  // 16-row groups of a tile: gate (and up)
   constexpr int G = G1 * TR;                           // 16-row groups: tile t, matrix g1 at t * G1 + g1
@@ -351,23 +352,23 @@ __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
   }
 }
 
-template <int NW, int MT, bool DUMP, int TR>
+template <int NW, bool DUMP, int TR>
 void by_mode_ks(int mode, const MfmaArgs& a, dim3 grid, hipStream_t st) {
-  constexpr int KB = MT >= 2 ? 1 : 2;  // small stages: occupancy (4-5 waves per SIMD) beats bytes per round
+  constexpr int KB = 2;  // small stages: occupancy (4-5 waves per SIMD) beats bytes per round
   if (mode == BTF_GEMV_STORE)
-    hipLaunchKernelGGL((gemm_ks_kernel<NW, MT, KB, BTF_GEMV_STORE, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((gemm_ks_kernel<NW, KB, BTF_GEMV_STORE, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
   else if (mode == BTF_GEMV_ADD)
-    hipLaunchKernelGGL((gemm_ks_kernel<NW, MT, KB, BTF_GEMV_ADD, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((gemm_ks_kernel<NW, KB, BTF_GEMV_ADD, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
   else
-    hipLaunchKernelGGL((gemm_ks_kernel<NW, MT, KB, BTF_GEMV_SWIGLU, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((gemm_ks_kernel<NW, KB, BTF_GEMV_SWIGLU, DUMP, TR>), grid, dim3(64 * NW), 0, st, a);
 }
 
-template <int MT, bool DUMP, int TR = 1>
+template <bool DUMP, int TR = 1>
 void by_waves_ks(int nw, int mode, const MfmaArgs& a, dim3 grid, hipStream_t st) {
   if (nw == 8)
-    by_mode_ks<8, MT, DUMP, TR>(mode, a, grid, st);
+    by_mode_ks<8, DUMP, TR>(mode, a, grid, st);
   else
-    by_mode_ks<4, MT, DUMP, TR>(mode, a, grid, st);
+    by_mode_ks<4, DUMP, TR>(mode, a, grid, st);
 }
 
 // The longest wave range (128-column blocks) the packed tile's preloads hold:
@@ -755,10 +756,8 @@ int mfma_rows_per_pass() { return 64; }
 int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
               hipStream_t st, const DevState&, const Q8* qout) {
   MfmaArgs a{};
-  if (nb > 32) {
-    if (qout) return fail(BTF_ERR_ARGS, "gemm: a Q8 output needs at most 32 rows");
-    return gemm_t32(segs, nseg, K, m0, nb, act, mode, dump, st);
-  }
+  if (qout && nb > 32) return fail(BTF_ERR_ARGS, "gemm: a Q8 output needs at most 32 rows");
+  if (nb > 16) return gemm_t32(segs, nseg, K, m0, nb, act, mode, dump, st, qout);
   // the K-split 16-row tile (32 rows with a Q8 output)
   if (qout && dump) return fail(BTF_ERR_ARGS, "gemm: a Q8 output has no dump");
   const int rows_real = qout ? 32 : 16;
@@ -795,43 +794,32 @@ int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& ac
     a.os = const_cast<int32_t*>(qout->s);
   }
   if (tiles == 0) return BTF_OK;
-  const int MT = nb <= 16 ? 1 : 2;
-  const int BM = 16 * MT;
-  const dim3 grid(tiles, (nb + BM - 1) / BM);
+  const dim3 grid(tiles, 1);
   const bool dmp = dump != nullptr;
-  // up to 16 rows with d and s 16-byte aligned (the LDS-direct loads of the
-  // packed tile read them in 16-byte pieces): the packed tile
+  // d and s 16-byte aligned (the LDS-direct loads of the packed tile read them
+  // in 16-byte pieces): the packed tile
   const int kw = kp_waves(K, mode);
-  if (nb <= 16 && kw && ((reinterpret_cast<uintptr_t>(act.d) | reinterpret_cast<uintptr_t>(act.s)) & 15) == 0) {
-    const dim3 gk(tiles, 1);
+  if (kw && ((reinterpret_cast<uintptr_t>(act.d) | reinterpret_cast<uintptr_t>(act.s)) & 15) == 0) {
     if (qout) {
       if (nb <= 8)
-        by_waves_kp<1, false, 2>(kw, mode, a, gk, st);
+        by_waves_kp<1, false, 2>(kw, mode, a, grid, st);
       else
-        by_waves_kp<2, false, 2>(kw, mode, a, gk, st);
+        by_waves_kp<2, false, 2>(kw, mode, a, grid, st);
     } else if (nb <= 8) {
-      dmp ? by_waves_kp<1, true>(kw, mode, a, gk, st) : by_waves_kp<1, false>(kw, mode, a, gk, st);
+      dmp ? by_waves_kp<1, true>(kw, mode, a, grid, st) : by_waves_kp<1, false>(kw, mode, a, grid, st);
     } else {
-      dmp ? by_waves_kp<2, true>(kw, mode, a, gk, st) : by_waves_kp<2, false>(kw, mode, a, gk, st);
+      dmp ? by_waves_kp<2, true>(kw, mode, a, grid, st) : by_waves_kp<2, false>(kw, mode, a, grid, st);
     }
     return launch_status("gemm_kp_kernel");
   }
-  // 8 waves split K for one activation tile (measured: down 29.6 -> 25.2 us and
-  // QKV 11.0 -> 10.1 us at M = 8), except gate+up at K = 5120 (27 -> 31 us);
-  // with two activation tiles 8 waves were slower on every shape
-  const int nw = MT == 1 && (K >= 8192 || mode != BTF_GEMV_SWIGLU) ? 8 : 4;
+  // 8 waves split K (measured: down 29.6 -> 25.2 us and QKV 11.0 -> 10.1 us at
+  // M = 8), except gate+up at K = 5120 (27 -> 31 us)
+  const int nw = K >= 8192 || mode != BTF_GEMV_SWIGLU ? 8 : 4;
   // (the K split depends on nw only: the outputs do not depend on the tile height)
-  if (qout) {
-    if (MT == 1)
-      by_waves_ks<1, false, 2>(nw, mode, a, grid, st);
-    else
-      by_waves_ks<2, false, 2>(nw, mode, a, grid, st);
-    return launch_status("gemm_ks_kernel");
-  }
-  if (MT == 1)
-    dmp ? by_waves_ks<1, true>(nw, mode, a, grid, st) : by_waves_ks<1, false>(nw, mode, a, grid, st);
+  if (qout)
+    by_waves_ks<false, 2>(nw, mode, a, grid, st);
   else
-    dmp ? by_waves_ks<2, true>(nw, mode, a, grid, st) : by_waves_ks<2, false>(nw, mode, a, grid, st);
+    dmp ? by_waves_ks<true>(nw, mode, a, grid, st) : by_waves_ks<false>(nw, mode, a, grid, st);
   return launch_status("gemm_ks_kernel");
 }
 

@@ -1,6 +1,6 @@
 // gemm_t32.hip -- ternary GEMM on T2 codes with 32x32 int8 MFMA tiles (gfx950),
-// for more than 32 activation rows (prefill). Same contract as the reference's
-// gemv_kernel (src/cuda/kernels.cu:238-334).
+// for more than 16 activation rows (larger decode batches, prefill). Same
+// contract as the reference's gemv_kernel (src/cuda/kernels.cu:238-334).
 //
 // What bounds it: the vector ALU. Every Q8 block has its own scale, so each
 // output takes an int32 -> fp32 conversion and a multiply-add per 32-column
@@ -30,7 +30,8 @@
 // group share the activation tile (32 MT rows, double-buffered in LDS, one
 // barrier a block) and own 32 staged weight rows each (swiglu: 16 gate rows and
 // the same 16 up rows). Per output the sums are blk = d * I over a block's
-// sub-blocks, then acc = scale * blk + acc per block.
+// sub-blocks, then acc = scale * blk + acc per block. For up to 32 rows (one
+// activation tile) the epilogue can also write the Q8 of the outputs.
 #include <climits>
 #include <type_traits>
 
@@ -64,6 +65,11 @@ struct T32Args {
   int m0, nb;
   int tn, tm;  // tiles along the outputs and the activation rows
   int32_t* dump;
+  // optional Q8 of the outputs (segment 0 after the mode), for the next GEMM:
+  // q [.][N], d and s [.][N / 32] at activation row m0 + m (one activation tile)
+  int8_t* oq;
+  float* od;
+  int32_t* os;
 };
 
 // LDS written by this workgroup visible to it; global loads stay in flight.
@@ -88,7 +94,9 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) g
   constexpr int SB = WN * 128;              // weight scales of a block: [staged row]
   constexpr int BUF = FB + DB + SB;
   constexpr int RED = (WK - 1) * WN * MT * 4096;
-  constexpr int LDS = 2 * WK * BUF > RED ? 2 * WK * BUF : RED;
+  constexpr int OUT = MT == 1 ? 32 * (BNR + 1) * 4 : 0;  // outputs to quantize: [activation row][output]
+  constexpr int LDS0 = 2 * WK * BUF > RED ? 2 * WK * BUF : RED;
+  constexpr int LDS = LDS0 > OUT ? LDS0 : OUT;
   __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
 
   const int tid = threadIdx.x;
@@ -301,6 +309,8 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) g
 
   // ---- epilogue (group 0): lane holds activation row mb + 32 i + l31; register r its
   // staged row 8 (r / 4) + 4 h + r % 4 (swiglu: gate rows in registers 0-7, their up rows in 8-15) ----
+  const bool quant = MT == 1 && a.oq;  // (uniform)
+  if (quant) lds_barrier();            // every read of the partial sums is done
   if (kg == 0) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -332,6 +342,35 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) g
           for (int r = 0; r < 4; ++r)
             if (n + r < N) yr[n + r] = MODE == BTF_GEMV_ADD ? yr[n + r] + v[r] : v[r];
         }
+        if (quant) {  // (N % 32 == 0: live blocks are whole)
+          float* ol = reinterpret_cast<float*>(lds) + l31 * (BNR + 1) + wn * TR + 8 * c + 4 * h;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) ol[r] = v[r];
+        }
+      }
+    }
+  }
+  if constexpr (MT == 1) {
+    if (quant) {
+      lds_barrier();
+      // a half-wave per (activation row, 32-output block), with the q8 kernel's arithmetic
+      const int b0 = (bx - tile0) * (BNR / 32), nblk = N / 32;
+      for (int e = 2 * w + h; e < 32 * (BNR / 32); e += 2 * WN * WK) {
+        const int mm = e & 31, bl = e >> 5;
+        float dq;
+        int sq;
+        const int q = q8_half(reinterpret_cast<const float*>(lds)[mm * (BNR + 1) + 32 * bl + l31], dq, sq);
+        uint32_t wq = (uint32_t)(q & 0xff) << (8 * (l31 & 3));
+        wq |= (uint32_t)dpp_i<0xB1>((int)wq);  // quad_perm(1,0,3,2)
+        wq |= (uint32_t)dpp_i<0x4E>((int)wq);  // quad_perm(2,3,0,1)
+        if (mb + mm < a.nb && b0 + bl < nblk) {
+          const size_t mr = (size_t)(a.m0 + mb + mm);
+          if ((l31 & 3) == 0) *reinterpret_cast<uint32_t*>(a.oq + mr * N + 32 * (b0 + bl) + l31) = wq;
+          if (l31 == 0) {
+            a.od[mr * nblk + b0 + bl] = dq;
+            a.os[mr * nblk + b0 + bl] = sq;
+          }
+        }
       }
     }
   }
@@ -353,7 +392,7 @@ void by_mode(int mode, const T32Args& a, int grid, hipStream_t st) {  // (a by r
 }  // namespace
 
 int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-             hipStream_t st) {
+             hipStream_t st, const Q8* qout) {
   T32Args a{};
   const int nuse = mode == BTF_GEMV_SWIGLU ? 1 : nseg;
   a.K = K;
@@ -366,6 +405,11 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   if (mode == BTF_GEMV_SWIGLU) {
     a.up_codes = segs[1].codes;
     a.up_scales = segs[1].scales;
+  }
+  if (qout) {
+    a.oq = const_cast<int8_t*>(qout->q);  // (Q8 holds read-only views; this one is written)
+    a.od = const_cast<float*>(qout->d);
+    a.os = const_cast<int32_t*>(qout->s);
   }
   // sets the n-tiles of `rows` output rows and the m-tiles of bm rows; returns the grid, which
   // covers 8 n-tiles at a time (see the kernel's mapping)
@@ -396,16 +440,19 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   // (17408 tiles) 2,4,1 233, 1,4,1 259, 1,2,4 300; 128 rows (4352) 1,4,1 82,
   // 2,4,1 84, 1,2,4 81; 64 rows (2176) 1,2,4 48, 1,4,1 51, 1,2,8 63; down
   // 17408 -> 5120, 203 rows (1120) 1,2,4 93, 1,4,1 117, 1,2,8 103; 5120 ->
-  // 5120, 64 rows (320) 1,2,8 14.0, 1,2,4 14.5, 1,4,1 28.
+  // 5120, 64 rows (320) 1,2,8 14.0, 1,2,4 14.5, 1,4,1 28; gate+up of 32 rows
+  // (1088) 1,2,4 34, 1,4,1 37, 1,2,8 42; 5120 -> 3 x 5120, 32 rows (480)
+  // 1,2,8 15.8, 1,2,4 16.6; 2048 -> 2 x 8192, 32 rows (512) 1,2,4 8.8, 1,2,8 9.8.
+  // (The choice does not depend on qout: y is the same with and without it.)
   const int per = mode == BTF_GEMV_SWIGLU ? 16 : 32;  // output rows of a wave
   tiles(per, 32);
   const int64_t t32 = (int64_t)a.tn * a.tm;
   if (t32 == 0) return BTF_OK;
-  if (t32 >= 8192)
+  if (t32 >= 8192 && nb > 32)
     by_mode<2, 4, 1>(mode, a, tiles(4 * per, 64), st);
   else if (t32 >= 4096)
     by_mode<1, 4, 1>(mode, a, tiles(4 * per, 32), st);
-  else if (t32 >= 640)
+  else if (t32 >= 500)
     by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
   else
     by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);

@@ -1,4 +1,4 @@
-"""The 32x32-tile GEMM (more than 32 activation rows) in each of its four tile
+"""The 32x32-tile GEMM (more than 16 activation rows) in each of its four tile
 shapes, at the edges of tiles, segments and K groups.
 
 Oracle: the exact int32 I of the oracle, scaled and summed in float64. An
@@ -51,6 +51,9 @@ def wide(oracle, mat, sel, K, q, d, s):
 
 # (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses
 CASES = [
+    (128, 17, [1, 33], 1),           # one activation tile with 15 dead rows
+    (256, 32, [16070, 5], 8030),     # 504 / 502 tiles: two waves x four groups, one full activation tile
+    (128, 25, [131105], 65600),      # 4098 / 4100 tiles of one activation tile: four waves, K unsplit
     (128, 33, [1, 33], 1),           # one block: seven of eight K groups have none
     (384, 64, [37, 70, 9], 17),      # three blocks over eight groups, three segments
     (1152, 95, [45], 50),            # nine blocks: uneven groups, a dead row in the last tile
@@ -114,3 +117,35 @@ def test_t32_modes_and_edges(hip, oracle, K, M, Ns, N2):
     I = torch.full((M, n, K // 32), -(1 << 30), dtype=torch.int32, device="cuda")
     hip.gemv_i32_dump(dev(mats[-1][0][:n]), n, K, M, act, I, stream())
     assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(np.ascontiguousarray(mats[-1][0][:n]), K, q, s))
+
+
+@pytest.mark.parametrize("K,M,N", [(128, 17, 64), (1152, 24, 96), (256, 32, 16064), (128, 30, 131136),
+                                   (128, 18, 262176)])
+def test_t32_q8_output(hip, oracle, K, M, N):
+    """launch_gemv_ex with a Q8 output in each tile shape of one activation
+    tile: y equals launch_gemv's bit for bit, the Q8 rows equal the oracle's
+    quantize of that y; the first block is all zero."""
+    torch = _torch()
+    rng = np.random.default_rng(K + M + N)
+    q, d, s = oracle.quantize_rows((rng.standard_normal((M, K)) * 2).astype(np.float32))
+    act = hip.Q8Act(dev(q), dev(d), dev(s))
+    mats = [matrix(rng, N, K) for _ in range(2)]
+    mats[0][0][:32] = 0x55  # trit 0
+    w = [(dev(c), dev(sc)) for c, sc in mats]
+    for mode in (hip.GemvMode.kStore, hip.GemvMode.kAdd, hip.GemvMode.kSwiglu):
+        ys = []
+        out = hip.Q8Act(torch.zeros((M, N), dtype=torch.int8, device="cuda"), torch.zeros((M, N // 32), device="cuda"),
+                        torch.zeros((M, N // 32), dtype=torch.int32, device="cuda"))
+        for fused in (False, True):
+            y = torch.zeros((M, N), device="cuda")
+            segs = [hip.GemvSeg(*w[0], N, y, N)] + ([hip.GemvSeg(*w[1], N, None, 0)] if mode == 2 else [])
+            if fused:
+                hip.launch_gemv_ex(segs, K, M, act, mode=mode, out=out, stream=stream())
+            else:
+                hip.launch_gemv(segs, K, M, act, mode, stream())
+            ys.append(y.cpu().numpy())
+        assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32)), f"y, mode {mode}"
+        rq, rd, rs = oracle.quantize_rows(ys[1])
+        assert np.array_equal(out.q.cpu().numpy(), rq), f"q, mode {mode}"
+        assert np.array_equal(out.d.cpu().numpy().view(np.uint32), rd.view(np.uint32)), f"d, mode {mode}"
+        assert np.array_equal(out.s.cpu().numpy(), rs), f"s, mode {mode}"
