@@ -16,17 +16,23 @@ from __future__ import annotations
 
 import ctypes as C
 import enum
+import importlib.util
 import os
 import sys
 from dataclasses import dataclass
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libbtf_hip.so")
+CALL_PATH = os.path.join(HERE, "_btf_call.so")
 
-if not os.path.exists(LIB_PATH):
-    raise ImportError(f"{LIB_PATH} is missing: build it with `make -C {HERE}` (hipcc, gfx950)")
+for _p in (LIB_PATH, CALL_PATH):
+    if not os.path.exists(_p):
+        raise ImportError(f"{_p} is missing: build it with `make -C {HERE}` (hipcc, gfx950)")
 
 _lib = C.CDLL(LIB_PATH)
+_spec = importlib.util.spec_from_file_location("_btf_call", CALL_PATH)
+_call = importlib.util.module_from_spec(_spec)
+_spec.loader.exec_module(_call)
 
 BTF_OK, BTF_ERR_ARGS, BTF_ERR_DEVICE, BTF_ERR_LAUNCH, BTF_ERR_NOT_INIT = 0, 1, 2, 3, 4
 
@@ -258,6 +264,12 @@ class GemvSeg:
         return _GemvSeg(_addr(self.codes), _addr(self.scales), self.N, _addr(self.y), self.ldy)
 
 
+# The launchers below go through the native calls of _btf_call; arguments that
+# those do not read (NotImplemented) take the ctypes path.
+_call.bind(*[C.cast(f, C.c_void_p).value for f in (_launch_prep, _launch_gemv, _launch_gemv_ptq1_0, _launch_gemv_ex)],
+           Q8Act, Hx, GemvSeg)
+
+
 def kernels_init(device: int = 0) -> None:
     """src/cuda/kernels.cuh:17"""
     _check(_kernels_init(device))
@@ -276,6 +288,11 @@ def launch_repack(src, nblocks: int, codes, scales, stream=None) -> None:
 def launch_prep(x, ldx: int, M: int, n: int, normw, eps: float, hx: Hx | None, xn_out, ldxn: int, a: Q8Act,
                 stream=None) -> None:
     """src/cuda/kernels.cuh:40-43"""
+    rc = _call.prep(x, ldx, M, n, normw, eps, hx, xn_out, ldxn, a, stream)
+    if rc is not NotImplemented:
+        if rc:
+            _check(rc)
+        return
     h = (hx or Hx())._c()
     q = a._c()
     _check(_launch_prep(_addr(x), ldx, M, n, _addr(normw), eps, C.byref(h), _addr(xn_out), ldxn, C.byref(q),
@@ -284,6 +301,11 @@ def launch_prep(x, ldx: int, M: int, n: int, normw, eps: float, hx: Hx | None, x
 
 def launch_gemv(segs, K: int, M: int, a: Q8Act, mode: GemvMode = GemvMode.kStore, stream=None) -> None:
     """src/cuda/kernels.cuh:53-56. `segs` is a list of 1..3 GemvSeg."""
+    rc = _call.gemv(segs, K, M, a, mode, stream)
+    if rc is not NotImplemented:
+        if rc:
+            _check(rc)
+        return
     arr = (_GemvSeg * max(1, len(segs)))(*[s._c() for s in segs])
     q = a._c()
     _check(_launch_gemv(arr, len(segs), K, M, C.byref(q), int(mode), _stream(stream)))
@@ -334,6 +356,11 @@ def launch_gemv_ex(segs, K: int, M: int, a: Q8Act = None, x=None, ldx: int = 0,
     """launch_gemv with the chain's quantizes fused in (no reference
     counterpart): input from Q8 rows `a` or fp32 rows `x` [M][ldx]; `out`
     (optional) receives the Q8 rows of the output."""
+    rc = _call.gemv_ex(segs, K, M, a, x, ldx, mode, out, stream)
+    if rc is not NotImplemented:
+        if rc:
+            _check(rc)
+        return
     _check(launch_gemv_ex_raw(segs, len(segs), K, M, a, x, ldx, int(mode), out, stream))
 
 
@@ -347,6 +374,11 @@ def launch_gemv_ex_raw(segs, nseg: int, K: int, M: int, a, x, ldx: int, mode: in
 def launch_gemv_ptq1_0(segs, K: int, M: int, a: Q8Act, mode: GemvMode = GemvMode.kStore, stream=None) -> None:
     """launch_gemv on PTQ1_0 matrices read directly: each GemvSeg's codes are
     N rows of K/128 28-byte PTQ1_0 blocks and its scales None."""
+    rc = _call.gemv_ptq1_0(segs, K, M, a, mode, stream)
+    if rc is not NotImplemented:
+        if rc:
+            _check(rc)
+        return
     _check(launch_gemv_ptq1_0_raw(segs, len(segs), K, M, a, int(mode), stream))
 
 
