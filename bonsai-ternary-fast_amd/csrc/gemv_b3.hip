@@ -11,7 +11,7 @@
 // consecutive bytes j..j+3 are four consecutive elements, and their dot4
 // operand is one activation word as stored.
 //
-// Decode (two bytes per 16-bit lane): t = q*3 (v_pk_mul_lo_u16) puts the
+// Decode (two bytes per 16-bit lane): t = q*3 puts the
 // digit in each lane's high byte and the next q in its low byte; one
 // v_perm_b32 gathers the high bytes of the two lanes of two words (bytes
 // j, j+2 and j+1, j+3) into the dot4 operand of bytes j..j+3. Per 4 weights:
@@ -56,11 +56,11 @@ struct B3Args {
   int m0, nb;
 };
 
-// k*v in each 16-bit lane
+// k*v in each 16-bit lane, for bytes v in lanes 0 and 1 and k <= 255: one
+// 24-bit multiply (the low product stays below 2^16), a 4-byte encoding where
+// the packed 16-bit multiply has 8 (output projection 77.5 -> 75.2 us)
 __device__ __forceinline__ uint32_t mulk(uint32_t v, uint16_t k) {
-  u16x2 x = __builtin_bit_cast(u16x2, v);
-  x = x * k;
-  return __builtin_bit_cast(uint32_t, x);
+  return __umul24(v, k);
 }
 // t = 3*v in each 16-bit lane
 __device__ __forceinline__ uint32_t mul3(uint32_t v) {
@@ -144,8 +144,8 @@ __device__ __forceinline__ void block_dot(const uint32_t (&w)[7], const uint32_t
   for (int k = 0; k < 4; ++k) I[k] = c.a[k] - 3 * c.b[k];
 }
 
-template <int NB, int T, int R, int MODE>
-__global__ void __launch_bounds__(1024) gemv_b3_kernel(B3Args a) {
+template <int NB, int T, int R, int MODE, int MAXT>
+__global__ void __launch_bounds__(MAXT) gemv_b3_kernel(B3Args a) {
   constexpr int RB = R * T;  // virtual rows per workgroup
   __shared__ float red[NB][kMaxSlices + 1][RB];
 
@@ -306,24 +306,24 @@ __global__ void __launch_bounds__(1024) gemv_b3_kernel(B3Args a) {
   }
 }
 
-template <int NB, int T, int R>
+template <int NB, int T, int R, int MAXT = 1024>
 void by_mode(int mode, const B3Args& a, int grid, int threads, hipStream_t st) {
   if (mode == BTF_GEMV_STORE)
-    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_STORE>), dim3(grid), dim3(threads), 0, st, a);
+    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_STORE, MAXT>), dim3(grid), dim3(threads), 0, st, a);
   else if (mode == BTF_GEMV_ADD)
-    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_ADD>), dim3(grid), dim3(threads), 0, st, a);
+    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_ADD, MAXT>), dim3(grid), dim3(threads), 0, st, a);
   else
-    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_SWIGLU>), dim3(grid), dim3(threads), 0, st, a);
+    hipLaunchKernelGGL((gemv_b3_kernel<NB, T, R, BTF_GEMV_SWIGLU, MAXT>), dim3(grid), dim3(threads), 0, st, a);
 }
 
-template <int NB, int R>
+template <int NB, int R, int MAXT = 1024>
 void by_t(int T, int mode, const B3Args& a, int grid, int threads, hipStream_t st) {
   if (T == 1)
-    by_mode<NB, 1, R>(mode, a, grid, threads, st);
+    by_mode<NB, 1, R, MAXT>(mode, a, grid, threads, st);
   else if (T == 2)
-    by_mode<NB, 2, R>(mode, a, grid, threads, st);
+    by_mode<NB, 2, R, MAXT>(mode, a, grid, threads, st);
   else
-    by_mode<NB, 4, R>(mode, a, grid, threads, st);
+    by_mode<NB, 4, R, MAXT>(mode, a, grid, threads, st);
 }
 
 }  // namespace
@@ -334,16 +334,26 @@ int gemv_b3(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act,
   const int nsl = (K + 1023) / 1024;
   if (nsl > kMaxSlices) return fail(BTF_ERR_ARGS, "gemv_ptq1_0: K must be at most 32768");
   if (nb < 1 || nb > 2) return fail(BTF_ERR_ARGS, "gemv_ptq1_0: 1 or 2 activation rows per pass");
-  // rows per step: 8 up to K = 16384 (one wave per slice), else 4
-  const int R = nsl <= 16 ? 8 : 4;
+  // rows per step: 8 up to K = 16384 (one wave per slice), else 4. Two activation
+  // rows: 4 from K > 12288, so that the workgroup has at most 768 threads (168
+  // registers) up to K = 24576
+  const int R = nsl <= (nb == 2 ? 12 : 16) ? 8 : 4;
   const int nw = (R * nsl + 7) / 8;
-  // keep >= 2 workgroups per CU
+  // Steps per workgroup (rows R T): every lane of a workgroup first loads its
+  // block's activation (136 bytes a row of it) for 28 T bytes of weights, so few
+  // steps make the launch L2-bound; fewer than 2 workgroups per CU leave it idle.
+  // With two activation rows the activation is twice as long and a half-filled
+  // chip is still the better one (T = 4 against 1, us: 5120 -> 5120, 160
+  // workgroups, 8.4 / 10.6; 5120 -> 2 x 17408 34 / 53; 17408 -> 5120 21 / 30; 5120 ->
+  // 248320 201 / 347; but 1024 -> 1024, 32 workgroups, 4.6 / 3.1). T = 8: slower at
+  // one row on every shape (5120 -> 248320 83 / 75).
   long rows = 0;
   for (int i = 0; i < nseg; ++i) rows += (mode == BTF_GEMV_SWIGLU && i > 0) ? 0 : segs[i].N;
   const int unit = mode == BTF_GEMV_SWIGLU ? R / 2 : R;
+  const long least = nb == 2 ? ds.cu_count / 2 : 2L * ds.cu_count;
   int T = 4;
-  while (T > 1 && rows / (unit * T) < 2L * ds.cu_count) T /= 2;
-  if (nb == 2) T = 1;  // register budget (two activation blocks per lane)
+  while (T > 1 && rows / (unit * T) < least) T /= 2;
+  if (nb == 2 && 64 * nw > 768) T = 1;  // (128 registers: one block of weights beside two of activation)
 
   B3Args a{};
   int wg = 0;
@@ -383,7 +393,9 @@ int gemv_b3(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act,
       by_t<1, 4>(T, mode, a, wg, threads, st);
   } else {
     if (R == 8)
-      by_mode<2, 1, 8>(mode, a, wg, threads, st);
+      by_t<2, 8, 768>(T, mode, a, wg, threads, st);
+    else if (threads <= 768)
+      by_t<2, 4, 768>(T, mode, a, wg, threads, st);
     else
       by_mode<2, 1, 4>(mode, a, wg, threads, st);
   }

@@ -185,3 +185,34 @@ def test_rejects_t2_arguments(hip):
         hip.launch_gemv_ptq1_0([hip.GemvSeg(blocks, sc, 4, y, 4)], 1024, 1, a, hip.GemvMode.kStore, stream())
     with pytest.raises(RuntimeError, match="32768"):
         hip.launch_gemv_ptq1_0([hip.GemvSeg(blocks, None, 4, y, 4)], 40960, 1, a, hip.GemvMode.kStore, stream())
+
+
+@pytest.mark.parametrize("K,N,mode", [(1024, 4099, "store"), (1024, 2100, "store"), (2048, 1030, "add"),
+                                      (1152, 2052, "swiglu"), (12288, 40, "store"), (12416, 2051, "add"),
+                                      (12416, 300, "swiglu"), (24576, 520, "store"), (24704, 33, "store")])
+def test_b3_two_rows_equal_one_row_launches(hip, K, N, mode):
+    """Two activation rows in one pass (4, 2 and 1 steps per workgroup, 8 and 4
+    rows a step, the largest workgroup) equal one-row launches bit for bit."""
+    import torch
+    rng = np.random.default_rng(K + N)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    nmat = 2 if mode == "swiglu" else 1
+    mats = []
+    for _ in range(nmat):
+        b = rng.integers(0, 256, (N, K // 128, 28), dtype=np.uint8)
+        b[..., 26:] = (0.01 + 0.04 * rng.random((N, K // 128, 1))).astype(np.float16).view(np.uint8)
+        mats.append(t(b))
+    q = rng.integers(-127, 128, (2, K)).astype(np.int8)
+    s = q.reshape(2, -1, 32).astype(np.int32).sum(-1).astype(np.int32)
+    d = (0.01 * rng.random((2, K // 32))).astype(np.float16).astype(np.float32)
+    y0 = rng.standard_normal((2, N)).astype(np.float32)
+    m = {"store": hip.GemvMode.kStore, "add": hip.GemvMode.kAdd, "swiglu": hip.GemvMode.kSwiglu}[mode]
+    st = torch.cuda.current_stream().cuda_stream
+
+    def run(rows):
+        y = t(y0[rows])
+        segs = [hip.GemvSeg(mats[0], None, N, y, N)] + ([hip.GemvSeg(mats[1], None, N)] if nmat == 2 else [])
+        hip.launch_gemv_ptq1_0(segs, K, len(rows), hip.Q8Act(t(q[rows]), t(d[rows]), t(s[rows])), m, st)
+        return y.cpu().numpy()
+    both, single = run([0, 1]), np.concatenate([run([0]), run([1])])
+    assert np.array_equal(both.view(np.uint32), single.view(np.uint32))
