@@ -132,7 +132,7 @@ __device__ __forceinline__ void quantize_lane(const float4 (&xv)[4 * CL], bool l
 }
 
 template <int CL, int NB, int T, int MODE, bool DUMP, bool QIN, bool QOUT>
-__global__ void __launch_bounds__(QOUT ? 640 : 1024) gemv_dot4_kernel(Dot4Args a) {
+__global__ void __launch_bounds__(QOUT || (CL == 2 && NB == 2) ? 640 : 1024) gemv_dot4_kernel(Dot4Args a) {
   constexpr int RB = 4 * T;  // virtual rows per workgroup (4 per step)
   __shared__ float red[NB][kMaxWaves * CL][RB];
   constexpr int kXW = CL * 320;  // QIN: LDS words per wave (q, d, s of its K range)
@@ -430,17 +430,18 @@ void qout_by_mode(int mode, const Dot4Args& a, int grid, int threads, hipStream_
     launch_one<CL, 1, 16, BTF_GEMV_SWIGLU, false, QIN, true>(a, grid, threads, st);
 }
 
-// Instantiated shapes: CL=1 with NB 1/2 (T 2/4/8) and NB 4 (T 2); CL=2 with
-// NB 1 (T 2/4). Every one of them fits 128 VGPRs without scratch.
+// Instantiated shapes: CL=1 with NB 1 (T 2/4/8), NB 2 (T 2/4) and NB 4 (T 2);
+// CL=2 with NB 1 (T 2/4) and, on at most 10 waves, NB 2 (T 2/4). None has
+// scratch; all but the last fit 128 VGPRs.
 template <int CL, int NB>
 void by_t(int T, int mode, bool dump, const Dot4Args& a, int grid, int threads, hipStream_t st) {
   if (dump) {
     by_mode<CL, NB, 2, true>(mode, a, grid, threads, st);
     return;
   }
-  if constexpr (CL * NB >= 4) {
+  if constexpr (CL == 1 && NB == 4) {
     by_mode<CL, NB, 2, false>(mode, a, grid, threads, st);
-  } else if constexpr (CL == 2) {
+  } else if constexpr (CL == 2 || NB == 2) {
     if (T == 2)
       by_mode<CL, NB, 2, false>(mode, a, grid, threads, st);
     else
@@ -465,7 +466,7 @@ int gemv_dot4(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& ac
   const int nw = (cpr + 16 * CL - 1) / (16 * CL);
   if (nw > kMaxWaves) return fail(BTF_ERR_ARGS, "gemv: K too large for the dot4 path");
   const int NB = nb <= 1 ? 1 : nb <= 2 ? 2 : 4;
-  if (CL * NB > 4 || (CL == 2 && NB > 1)) return fail(BTF_ERR_ARGS, "gemv: batch too large for the dot4 path");
+  if (CL * NB > 4 || (CL == 2 && (NB > 2 || (NB == 2 && nw > 10)))) return fail(BTF_ERR_ARGS, "gemv: batch too large for the dot4 path");
   if ((x || qout) && (nb != 1 || dump)) return fail(BTF_ERR_ARGS, "gemv: the fused quantizes take one row");
   if (qout && nw > 10) return fail(BTF_ERR_ARGS, "gemv: the fused output quantize takes K <= 20480");
   if (qout && CL == 2 && mode == BTF_GEMV_SWIGLU)
@@ -476,9 +477,13 @@ int gemv_dot4(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& ac
   long rows = 0;
   for (int i = 0; i < nseg; ++i) rows += (mode == BTF_GEMV_SWIGLU && i > 0) ? 0 : segs[i].N;
   int T = 8;
-  while (T > 2 && rows / (unit * T) < 2L * ds.cu_count) T /= 2;
-  if (NB * CL >= 4 && T > 2) T = 2;  // register budget
+  const long least = NB == 2 && CL == 2 ? ds.cu_count : 2L * ds.cu_count;  // (17408 -> 5120: T = 4 16.0 us, T = 2 16.8)
+  while (T > 2 && rows / (unit * T) < least) T /= 2;
+  if (NB * CL >= 4 && CL == 1 && T > 2) T = 2;  // register budget
   if (CL == 2 && T > 4) T = 4;
+  // two rows: 84 registers (5 waves per SIMD) at T = 4, 104 (4) at T = 8: gate+up
+  // 15.8 against 18.4 us, output projection 83 against 93
+  if (NB == 2 && T > 4) T = 4;
   if (dump) T = 2;
   if (qout) T = mode == BTF_GEMV_SWIGLU ? 16 : 8;  // one 32-row output block per workgroup
 
@@ -540,7 +545,8 @@ int gemv_dot4(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& ac
     else if (NB == 2) by_t<1, 2>(T, mode, dmp, a, wg, threads, st);
     else by_t<1, 4>(T, mode, dmp, a, wg, threads, st);
   } else {
-    by_t<2, 1>(T, mode, dmp, a, wg, threads, st);
+    if (NB == 1) by_t<2, 1>(T, mode, dmp, a, wg, threads, st);
+    else by_t<2, 2>(T, mode, dmp, a, wg, threads, st);
   }
   return launch_status("gemv_dot4_kernel");
 }

@@ -149,3 +149,28 @@ def test_t32_q8_output(hip, oracle, K, M, N):
         assert np.array_equal(out.q.cpu().numpy(), rq), f"q, mode {mode}"
         assert np.array_equal(out.d.cpu().numpy().view(np.uint32), rd.view(np.uint32)), f"d, mode {mode}"
         assert np.array_equal(out.s.cpu().numpy(), rs), f"s, mode {mode}"
+
+
+@pytest.mark.parametrize("K,N", [(1024, 2053), (1024, 1030), (5120, 33), (16384, 40), (16512, 2055), (16512, 4100),
+                                 (17408, 20), (20480, 35), (20608, 18)])
+def test_dot4_two_rows_equal_one_row_launches(hip, oracle, K, N):
+    """Two activation rows on the v_dot4 path in one pass (both step counts,
+    one and two chunks per lane, the widest rows one pass takes and the next
+    wider) equal one-row launches bit for bit, and I equals the oracle's."""
+    torch = _torch()
+    rng = np.random.default_rng(K + N)
+    q, d, s = oracle.quantize_rows((rng.standard_normal((2, K)) * 2).astype(np.float32))
+    mats = [matrix(rng, N, K) for _ in range(2)]
+    w = [(dev(c), dev(sc)) for c, sc in mats]
+    y0 = rng.standard_normal((2, N)).astype(np.float32)
+    for mode in (hip.GemvMode.kStore, hip.GemvMode.kAdd, hip.GemvMode.kSwiglu):
+        def run(rows):
+            y = dev(y0[rows])
+            segs = [hip.GemvSeg(*w[0], N, y, N)] + ([hip.GemvSeg(*w[1], N, None, 0)] if mode == 2 else [])
+            hip.launch_gemv(segs, K, len(rows), hip.Q8Act(dev(q[rows]), dev(d[rows]), dev(s[rows])), mode, stream())
+            return y.cpu().numpy()
+        both, single = run([0, 1]), np.concatenate([run([0]), run([1])])
+        assert np.array_equal(both.view(np.uint32), single.view(np.uint32)), f"mode {mode}"
+    I = torch.zeros((2, N, K // 32), dtype=torch.int32, device="cuda")
+    hip.gemv_i32_dump(w[0][0], N, K, 2, hip.Q8Act(dev(q), dev(d), dev(s)), I, stream())
+    assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(mats[0][0], K, q, s))
