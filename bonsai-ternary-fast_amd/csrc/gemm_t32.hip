@@ -80,7 +80,7 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 template <int MT, int WN, int WK, int MODE, bool DUMP>
-__global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) gemm_t32_kernel(T32Args a) {
+__global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_t32_kernel(T32Args a) {
   constexpr bool SW = MODE == BTF_GEMV_SWIGLU;
   constexpr int BM = 32 * MT;               // activation rows
   constexpr int TR = SW ? 16 : 32;          // output rows of a 32-row weight tile (swiglu: 16 gate + their 16 up rows)
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) g
   constexpr int DB = BM * 4 * 4;            // d of a block: [sub-block][row]
   constexpr int SB = WN * 128;              // weight scales of a block: [staged row]
   constexpr int BUF = FB + DB + SB;
-  constexpr int RED = (WK - 1) * WN * MT * 4096;
+  constexpr int RED = WK > 1 ? WK * WN * MT * 4096 : 0;
   constexpr int OUT = MT == 1 ? 32 * (BNR + 1) * 4 : 0;  // outputs to quantize: [activation row][output]
   constexpr int LDS0 = 2 * WK * BUF > RED ? 2 * WK * BUF : RED;
   constexpr int LDS = LDS0 > OUT ? LDS0 : OUT;
@@ -286,69 +286,85 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 ? 4 : MT == 2 ? 3 : 2) g
   }
   if constexpr (DUMP) return;
 
-  // ---- the groups' partial sums, added in group order by group 0 ----
-  if constexpr (WK > 1) {
-    float* red = reinterpret_cast<float*>(lds);  // [kg - 1][wn][tile][register][lane] (over the buffers: all reads are done)
-    if (kg > 0) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) red[((((kg - 1) * WN + wn) * MT + i) * 16 + r) * 64 + lane] = acc[i][r];
-    }
-    lds_barrier();
-    if (kg == 0) {
-#pragma unroll
-      for (int g = 1; g < WK; ++g)
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            acc[i][r] = acc[i][r] + red[((((g - 1) * WN + wn) * MT + i) * 16 + r) * 64 + lane];
-    }
-  }
-
-  // ---- epilogue (group 0): lane holds activation row mb + 32 i + l31; register r its
-  // staged row 8 (r / 4) + 4 h + r % 4 (swiglu: gate rows in registers 0-7, their up rows in 8-15) ----
+  // ---- epilogue: lane holds activation row mb + 32 i + l31; register r its staged row
+  // 8 (r / 4) + 4 h + r % 4 (swiglu: gate rows in registers 0-7, their up rows in 8-15),
+  // so four registers (a chunk c) are four consecutive outputs ----
   const bool quant = MT == 1 && a.oq;  // (uniform)
-  if (quant) lds_barrier();            // every read of the partial sums is done
-  if (kg == 0) {
+  auto emit = [&](int i, int c, const f32x4& g, const f32x4& u) {
+    const int m = mb + 32 * i + l31;
+    const bool live = m < a.nb;
+    float* yr = y + (size_t)(a.m0 + (live ? m : 0)) * ldy;
+    const int n = n0 + 8 * c + 4 * h;
+    f32x4u v;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int m = mb + 32 * i + l31;
-      const bool live = m < a.nb;
-      float* yr = y + (size_t)(a.m0 + (live ? m : 0)) * ldy;
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (SW)
+        v[r] = g[r] / (1.0f + expf(-g[r])) * u[r];
+      else
+        v[r] = g[r];
+    }
+    if (live && n + 3 < N) {
+      f32x4u* o = reinterpret_cast<f32x4u*>(yr + n);
+      if constexpr (MODE == BTF_GEMV_ADD) {
+        const f32x4u old = *o;
 #pragma unroll
-      for (int c = 0; c < (SW ? 2 : 4); ++c) {
-        const int n = n0 + 8 * c + 4 * h;
-        f32x4u v;
+        for (int r = 0; r < 4; ++r) v[r] = old[r] + v[r];
+      }
+      *o = v;
+    } else if (live) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float g = acc[i][4 * c + r];
-          if constexpr (SW)
-            v[r] = g / (1.0f + expf(-g)) * acc[i][4 * c + r + 8];
-          else
-            v[r] = g;
-        }
-        if (live && n + 3 < N) {
-          f32x4u* o = reinterpret_cast<f32x4u*>(yr + n);
-          if constexpr (MODE == BTF_GEMV_ADD) {
-            const f32x4u old = *o;
+      for (int r = 0; r < 4; ++r)
+        if (n + r < N) yr[n + r] = MODE == BTF_GEMV_ADD ? yr[n + r] + v[r] : v[r];
+    }
+    if (quant) {  // (N % 32 == 0: live blocks are whole)
+      float* ol = reinterpret_cast<float*>(lds) + l31 * (BNR + 1) + wn * TR + 8 * c + 4 * h;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = old[r] + v[r];
+      for (int r = 0; r < 4; ++r) ol[r] = v[r];
+    }
+  };
+  constexpr int NC = SW ? 2 : 4;  // chunks of outputs
+  auto chunk = [&](int i, int c) { return f32x4{acc[i][4 * c], acc[i][4 * c + 1], acc[i][4 * c + 2], acc[i][4 * c + 3]}; };
+  if constexpr (WK > 1) {
+    // The groups' partial sums, added in group order: group c adds and writes
+    // chunk c, so a lane reads WK 16-byte words (swiglu: twice that) in a row
+    // and not, as one group adding them all would, 16 (WK - 1) registers.
+    static_assert(WK >= NC, "a group per chunk");
+    f32x4* red = reinterpret_cast<f32x4*>(lds);  // [kg][wn][tile][chunk][lane] (over the buffers: all reads are done)
+    auto slot = [&](int g, int i, int c) { return (((g * WN + wn) * MT + i) * 4 + c) * 64 + lane; };
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) red[slot(kg, i, c)] = chunk(i, c);
+    lds_barrier();
+    f32x4 g[MT], u[MT];
+    if (kg < NC) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        g[i] = red[slot(0, i, kg)];
+        if constexpr (SW) u[i] = red[slot(0, i, kg + 2)];
+#pragma unroll
+        for (int k = 1; k < WK; ++k) {
+          const f32x4 gk = red[slot(k, i, kg)];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) g[i][r] = g[i][r] + gk[r];
+          if constexpr (SW) {
+            const f32x4 uk = red[slot(k, i, kg + 2)];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u[i][r] = u[i][r] + uk[r];
           }
-          *o = v;
-        } else if (live) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < N) yr[n + r] = MODE == BTF_GEMV_ADD ? yr[n + r] + v[r] : v[r];
-        }
-        if (quant) {  // (N % 32 == 0: live blocks are whole)
-          float* ol = reinterpret_cast<float*>(lds) + l31 * (BNR + 1) + wn * TR + 8 * c + 4 * h;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ol[r] = v[r];
         }
       }
     }
+    if (quant) lds_barrier();  // every read of the partial sums is done
+    if (kg < NC) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) emit(i, kg, g[i], u[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) emit(i, c, chunk(i, c), SW ? chunk(i, c + 2) : f32x4{});
   }
   if constexpr (MT == 1) {
     if (quant) {
@@ -440,22 +456,40 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   // (17408 tiles) 2,4,1 233, 1,4,1 259, 1,2,4 300; 128 rows (4352) 1,4,1 82,
   // 2,4,1 84, 1,2,4 81; 64 rows (2176) 1,2,4 48, 1,4,1 51, 1,2,8 63; down
   // 17408 -> 5120, 203 rows (1120) 1,2,4 93, 1,4,1 117, 1,2,8 103; 5120 ->
-  // 5120, 64 rows (320) 1,2,8 14.0, 1,2,4 14.5, 1,4,1 28; gate+up of 32 rows
-  // (1088) 1,2,4 34, 1,4,1 37, 1,2,8 42; 5120 -> 3 x 5120, 32 rows (480)
-  // 1,2,8 15.8, 1,2,4 16.6; 2048 -> 2 x 8192, 32 rows (512) 1,2,4 8.8, 1,2,8 9.8.
-  // (The choice does not depend on qout: y is the same with and without it.)
+  // 5120, 64 rows (320) 1,2,8 13.4, 1,2,4 14.0, 1,1,4 15.6; gate+up of 32 rows
+  // (1088) 1,2,4 34, 1,4,1 37, 1,2,8 41; 5120 -> 3 x 5120, 32 rows (480)
+  // 1,2,8 15.8, 1,2,4 16.2; 2048 -> 2 x 2048, 96 rows (384) 1,2,4 7.7, 1,2,8
+  // 8.7. At most one tile per CU: a workgroup of one tile, on as many CUs as
+  // there are tiles; 32 rows, 5120 -> 5120 (160) 1,1,8 9.7, 1,2,8 12.8, 1,1,4
+  // 11.4; down (160) 1,1,12 27.4, 1,1,8 28.8, 1,2,8 36; 4096 -> 2048 (64) 1,1,8
+  // 7.8, 1,1,12 8.1, 1,2,8 10.5; 1024 -> 1024 (32) 1,1,4 4.22, 1,1,8 4.22, 1,2,8
+  // 5.4; one block per group: 512 -> 3 x 4096, 64 rows (768) 1,1,4 5.0, 1,2,4 5.5.
+  // (qout does not change the K split: y is the same with and without it.)
   const int per = mode == BTF_GEMV_SWIGLU ? 16 : 32;  // output rows of a wave
   tiles(per, 32);
   const int64_t t32 = (int64_t)a.tn * a.tm;
   if (t32 == 0) return BTF_OK;
-  if (t32 >= 8192 && nb > 32)
+  if (t32 >= 8192 && nb > 32) {
     by_mode<2, 4, 1>(mode, a, tiles(4 * per, 64), st);
-  else if (t32 >= 4096)
+  } else if (t32 >= 4096) {
     by_mode<1, 4, 1>(mode, a, tiles(4 * per, 32), st);
-  else if (t32 >= 500)
+  } else if (t32 <= 256 || (K <= 512 && t32 < 1024)) {
+    // (a swiglu's Q8 blocks are two waves wide: the same K split, so the same y)
+    const bool wide = qout && mode == BTF_GEMV_SWIGLU;
+    if (K <= 1024) {
+      if (wide) by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
+      else by_mode<1, 1, 4>(mode, a, tiles(per, 32), st);
+    } else if (K < 12288 || mode == BTF_GEMV_SWIGLU) {
+      if (wide) by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);
+      else by_mode<1, 1, 8>(mode, a, tiles(per, 32), st);
+    } else {
+      by_mode<1, 1, 12>(mode, a, tiles(per, 32), st);
+    }
+  } else if (t32 >= 500 || K < 4096) {
     by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
-  else
+  } else {
     by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);
+  }
   return launch_status("gemm_t32_kernel");
 }
 

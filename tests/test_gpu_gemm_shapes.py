@@ -1,4 +1,4 @@
-"""The 32x32-tile GEMM (more than 16 activation rows) in each of its four tile
+"""The 32x32-tile GEMM (more than 16 activation rows) in each of its tile
 shapes, at the edges of tiles, segments and K groups.
 
 Oracle: the exact int32 I of the oracle, scaled and summed in float64. An
@@ -51,13 +51,17 @@ def wide(oracle, mat, sel, K, q, d, s):
 
 # (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses
 CASES = [
-    (128, 17, [1, 33], 1),           # one activation tile with 15 dead rows
-    (256, 32, [16070, 5], 8030),     # 504 / 502 tiles: two waves x four groups, one full activation tile
+    (128, 17, [1, 33], 1),           # one activation tile with 15 dead rows, one block: three of four K groups have none
+    (256, 32, [16070, 5], 8030),     # 504 / 502 tiles of few blocks: one wave x four groups, one full activation tile
     (128, 25, [131105], 65600),      # 4098 / 4100 tiles of one activation tile: four waves, K unsplit
-    (128, 33, [1, 33], 1),           # one block: seven of eight K groups have none
-    (384, 64, [37, 70, 9], 17),      # three blocks over eight groups, three segments
-    (1152, 95, [45], 50),            # nine blocks: uneven groups, a dead row in the last tile
+    (384, 64, [37, 70, 9], 17),      # three blocks over four groups, three segments
+    (1152, 95, [45], 50),            # one wave x eight groups, nine blocks: uneven groups, a dead row in the last tile
+    (1152, 32, [8161], 4081),        # 256 / 256 tiles: the last of one tile per workgroup
+    (1152, 32, [8193], 4097),        # 257 / 257 tiles: two waves x four groups
+    (12416, 40, [37, 5], 20),        # one wave x twelve groups (swiglu: eight), 97 blocks
+    (4224, 64, [4200], 2200),        # 264 / 276 tiles: two waves x eight groups, 33 blocks
     (640, 65, [6917], 3500),         # 651 / 657 tiles: two waves x four groups; five blocks
+    (640, 32, [16070, 5], 8030),     # the same of one full activation tile
     (256, 200, [18733], 9400),       # 4102 / 4116 tiles: four waves, K unsplit
     (256, 513, [15500], 7800),       # 8245 / 8296 tiles: 64 activation rows a wave, the last tile nearly empty
 ]
@@ -119,7 +123,8 @@ def test_t32_modes_and_edges(hip, oracle, K, M, Ns, N2):
     assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(np.ascontiguousarray(mats[-1][0][:n]), K, q, s))
 
 
-@pytest.mark.parametrize("K,M,N", [(128, 17, 64), (1152, 24, 96), (256, 32, 16064), (128, 30, 131136),
+@pytest.mark.parametrize("K,M,N", [(128, 17, 64), (1152, 24, 96), (12416, 20, 64), (4224, 20, 8480),
+                                   (1152, 32, 8224), (256, 32, 16064), (128, 30, 131136),
                                    (128, 18, 262176)])
 def test_t32_q8_output(hip, oracle, K, M, N):
     """launch_gemv_ex with a Q8 output in each tile shape of one activation
