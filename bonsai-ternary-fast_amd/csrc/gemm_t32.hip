@@ -464,6 +464,9 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   // 11.4; down (160) 1,1,12 27.4, 1,1,8 28.8, 1,2,8 36; 4096 -> 2048 (64) 1,1,8
   // 7.8, 1,1,12 8.1, 1,2,8 10.5; 1024 -> 1024 (32) 1,1,4 4.22, 1,1,8 4.22, 1,2,8
   // 5.4; one block per group: 512 -> 3 x 4096, 64 rows (768) 1,1,4 5.0, 1,2,4 5.5.
+  // K unsplit from 3000 tiles: 3072 -> 3072, 1000 rows (3072) 1,4,1 37, 1,2,4 40;
+  // and from 1024 where a group would have at most one block: 256 -> 3 x 2048,
+  // 512 rows (3072) 1,4,1 7.2, 1,2,4 12.4.
   // (qout does not change the K split: y is the same with and without it.)
   const int per = mode == BTF_GEMV_SWIGLU ? 16 : 32;  // output rows of a wave
   tiles(per, 32);
@@ -471,7 +474,7 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   if (t32 == 0) return BTF_OK;
   if (t32 >= 8192 && nb > 32) {
     by_mode<2, 4, 1>(mode, a, tiles(4 * per, 64), st);
-  } else if (t32 >= 4096) {
+  } else if (t32 >= 3000 || (K <= 512 && t32 >= 1024)) {
     by_mode<1, 4, 1>(mode, a, tiles(4 * per, 32), st);
   } else if (t32 <= 256 || (K <= 512 && t32 < 1024)) {
     // (a swiglu's Q8 blocks are two waves wide: the same K split, so the same y)

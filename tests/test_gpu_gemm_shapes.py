@@ -62,6 +62,8 @@ CASES = [
     (4224, 64, [4200], 2200),        # 264 / 276 tiles: two waves x eight groups, 33 blocks
     (640, 65, [6917], 3500),         # 651 / 657 tiles: two waves x four groups; five blocks
     (640, 32, [16070, 5], 8030),     # the same of one full activation tile
+    (512, 520, [2000], 1000),        # 1071 / 1071 tiles of few blocks: four waves, K unsplit
+    (1152, 1000, [3000], 1500),      # 3008 / 3008 tiles: four waves, K unsplit
     (256, 200, [18733], 9400),       # 4102 / 4116 tiles: four waves, K unsplit
     (256, 513, [15500], 7800),       # 8245 / 8296 tiles: 64 activation rows a wave, the last tile nearly empty
 ]
