@@ -8,8 +8,8 @@
 // x 32 activation rows) comes with 32 such instructions and, measured on
 // independent instructions, 110 cycles of a SIMD at 4 waves (118 at 2, 176 at
 // one), 21 of them the MFMA's. At gate+up of 512 rows (5120 -> 2 x 17408) the
-// kernel holds the vector ALU 94 % of the time (SQ counters) and takes 233 us,
-// against 290 for the 16x16x32 tile it replaced, from:
+// kernel holds the vector ALU 93 % of the time (SQ counters) and takes 240 us,
+// against 280 for the 16x16x32 tile it replaced, from:
 //  - the weights as the MFMA's row operand: a lane's outputs then belong to one
 //    activation row, so d is one register per sub-block instead of four, and a
 //    lane stores four consecutive outputs at a time;
@@ -18,7 +18,7 @@
 //  - LDS addresses that are a register plus a constant (the loop body is
 //    written for both buffers) and weight scales converted when they are
 //    staged: 14 additions and 32 mixed-precision multiply-adds a block less
-//    (252 -> 233 us);
+//    (252 -> 233 us, K in one sum);
 //  - step e + 1's MFMA and step e + 2's LDS reads issued before step e is scaled.
 // The other ways to the float sums cost the same or more: adding 1.5 * 2^23
 // through the accumulator and subtracting it (115-128 cycles a step), and
@@ -26,7 +26,7 @@
 // be converted for every workgroup).
 //
 // A workgroup is WK groups of WN waves. The groups split the 128-column blocks
-// of K (contiguous shares, added in group order at the end); the waves of a
+// of K (contiguous parts, added in order at the end); the waves of a
 // group share the activation tile (32 MT rows, double-buffered in LDS, one
 // barrier a block) and own 32 staged weight rows each (swiglu: 16 gate rows and
 // the same 16 up rows). Per output the sums are blk = d * I over a block's
@@ -49,6 +49,20 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // y rows have any 4-byte alignment
+
+// The order of the sums. K is cut into G contiguous shares of its 128-column
+// blocks: share g is blocks nsc g / G .. nsc (g + 1) / G, summed in order from
+// zero, and the shares are added in order. G follows from the matrix alone and
+// every tile shape keeps to it, so an output of more than 16 rows has the same
+// bits whatever the launch's rows, segments and mode are. A tile that splits K
+// over fewer groups than G sets the sums of each share aside in LDS.
+// G is 8 where a launch of few rows splits K over 8 groups of waves (32 rows,
+// us, 4 groups / 8: 3072 -> 3072 7.5 / 6.6, 5120 -> 5120 11.2 / 9.5), and 4 where
+// that gains little (2048 -> 2048 5.9 / 5.6) or nothing (16384 outputs and more
+// fill the chip by themselves), because a tile that does not split K pays for each
+// share: gate+up of 512 rows (5120 -> 2 x 17408) 238 us with all of K in one
+// sum, 244 in 4 shares, 249 in 8; 2048 -> 2 x 8192, 512 rows, 49.5, 52.6, 55.3.
+__host__ __device__ constexpr int k_shares_log2(int nsc, int N) { return nsc <= 16 || N >= 16384 ? 2 : 3; }
 
 struct T32Args {
   const uint8_t* codes[3];
@@ -93,16 +107,19 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
   constexpr int DB = BM * 4 * 4;            // d of a block: [sub-block][row]
   constexpr int SB = WN * 128;              // weight scales of a block: [staged row]
   constexpr int BUF = FB + DB + SB;
-  constexpr int RED = WK > 1 ? WK * WN * MT * 4096 : 0;
+  constexpr int MS = WK == 1 ? 8 : WN == 2 ? 8 / WK : 1;  // the most shares of K that a group holds
+  constexpr int PART = WN * MT * 4096;      // a group's sums: [tile, chunk][thread]
+  constexpr int SAVE = MS > 1 && !DUMP ? PART : 0;  // those of the shares before its last one
+  constexpr int GRP = 2 * BUF + SAVE;       // LDS of a group
   constexpr int OUT = MT == 1 ? 32 * (BNR + 1) * 4 : 0;  // outputs to quantize: [activation row][output]
-  constexpr int LDS0 = 2 * WK * BUF > RED ? 2 * WK * BUF : RED;
-  constexpr int LDS = LDS0 > OUT ? LDS0 : OUT;
+  constexpr int LDS = WK * GRP > OUT ? WK * GRP : OUT;
+  static_assert(WK == 1 || PART <= 2 * BUF, "the partial sums go over the buffers");
   __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = w % WN, kg = w / WN;
+  const int wn = w % WN, kg = WK == 1 ? 0 : w / WN;
   const int tg = tid - kg * TG;  // thread within the group
   const int l31 = lane & 31, h = lane >> 5;
 
@@ -125,7 +142,7 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
   const int n0 = (bx - tile0) * BNR + wn * TR;  // this wave's first output row
   const int k0 = nsc * kg / WK, k1 = nsc * (kg + 1) / WK;
   const int niter = (nsc + WK - 1) / WK;  // the same for every group (barriers)
-  uint8_t* buf = lds + kg * 2 * BUF;
+  uint8_t* buf = lds + kg * GRP;
 
   // ---- load sources ----
   const uint8_t* csrc;   // codes: staged row l31, words 4h .. 4h + 3 of a block
@@ -187,6 +204,39 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
   v16i zero;
 #pragma unroll
   for (int r = 0; r < 16; ++r) zero[r] = 0;
+  // This thread's 16-byte slot for chunk c of activation tile i in a part of PART bytes. Its
+  // offset takes no register of the loop: one group has it in its first q offset, more
+  // compute it anew from the thread id (a value the compiler keeps spills in <1,2,4>).
+  auto slot = [&](uint8_t* part, int i, int c) -> f32x4& {
+    int off;
+    if constexpr (WK == 1) {
+      off = (int)qdst[0];
+    } else {
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+      off = 16 * (t - kg * TG);
+    }
+    return *reinterpret_cast<f32x4*>(part + off + (4 * i + c) * 16 * TG);
+  };
+  auto saved = [&](int g, int i, int c) -> f32x4& { return slot(lds + g * GRP + 2 * BUF, i, c); };
+  auto partial = [&](int g, int i, int c) -> f32x4& { return slot(lds + g * GRP, i, c); };
+  // G = 2^lg (one share a group: the launch takes the tile only where G is WK)
+  const int lg = MS > 1 ? k_shares_log2(nsc, N) : WK == 8 ? 3 : 2;
+  int sh = (kg << lg) / WK, kend = nsc * (sh + 1) >> lg;  // the share that holds the next block, and its end
+  while (kend <= k0 && kend < k1) kend = nsc * (++sh + 1) >> lg;  // (shares of short rows can be empty)
+  bool kept = false;  // a share's sums are in `saved`
+  auto chunk = [&](int i, int c) { return f32x4{acc[i][4 * c], acc[i][4 * c + 1], acc[i][4 * c + 2], acc[i][4 * c + 3]}; };
+  auto add_saved = [&] {  // acc = saved + acc, the reads all in flight together
+    f32x4 o[MT][4];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[i][c] = saved(0, i, c);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][r] = o[i][r >> 2][r & 3] + acc[i][r];
+  };
 
   if (k0 < k1) {
     fetch_act(k0);
@@ -277,6 +327,22 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (MS > 1 && !DUMP) {
+        if (kb + 1 == kend && kend < k1) {  // the share ends here, and the group has another one
+          if (WK == 1 && kept) add_saved();  // (a group that holds all of K adds its shares as it goes)
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              saved(kg, i, c) = chunk(i, c);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[i][4 * c + r] = 0.f;
+            }
+          kept = true;
+          do kend = nsc * (++sh + 1) >> lg;
+          while (kend <= kb + 1);
+        }
+      }
     }
     lds_barrier();
   };
@@ -323,36 +389,46 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
     }
   };
   constexpr int NC = SW ? 2 : 4;  // chunks of outputs
-  auto chunk = [&](int i, int c) { return f32x4{acc[i][4 * c], acc[i][4 * c + 1], acc[i][4 * c + 2], acc[i][4 * c + 3]}; };
   if constexpr (WK > 1) {
-    // The groups' partial sums, added in group order: group c adds and writes
-    // chunk c, so a lane reads WK 16-byte words (swiglu: twice that) in a row
+    // The groups' sums, added in share order: group c adds and writes
+    // chunk c, so a lane reads G 16-byte words (swiglu: twice that) in a row
     // and not, as one group adding them all would, 16 (WK - 1) registers.
-    static_assert(WK >= NC, "a group per chunk");
-    f32x4* red = reinterpret_cast<f32x4*>(lds);  // [kg][wn][tile][chunk][lane] (over the buffers: all reads are done)
-    auto slot = [&](int g, int i, int c) { return (((g * WN + wn) * MT + i) * 4 + c) * 64 + lane; };
+    static_assert(WK >= NC && MS <= 2, "a group per chunk");
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) red[slot(kg, i, c)] = chunk(i, c);
+      for (int c = 0; c < 4; ++c) partial(kg, i, c) = chunk(i, c);  // (over the buffers: all reads are done)
     lds_barrier();
     f32x4 g[MT], u[MT];
     if (kg < NC) {
+      auto total = [&](int i, int c) {
+        f32x4 p[WK], t;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        g[i] = red[slot(0, i, kg)];
-        if constexpr (SW) u[i] = red[slot(0, i, kg + 2)];
+        for (int k = 0; k < WK; ++k) p[k] = partial(k, i, c);
+        if (kept) {  // two shares a group (of 17 blocks and more: none is empty)
+          f32x4 v[WK];
 #pragma unroll
-        for (int k = 1; k < WK; ++k) {
-          const f32x4 gk = red[slot(k, i, kg)];
+          for (int k = 0; k < WK; ++k) v[k] = saved(k, i, c);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) g[i][r] = g[i][r] + gk[r];
-          if constexpr (SW) {
-            const f32x4 uk = red[slot(k, i, kg + 2)];
+          for (int r = 0; r < 4; ++r) {
+            t[r] = v[0][r] + p[0][r];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) u[i][r] = u[i][r] + uk[r];
+            for (int k = 1; k < WK; ++k) t[r] = (t[r] + v[k][r]) + p[k][r];
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            t[r] = p[0][r];
+#pragma unroll
+            for (int k = 1; k < WK; ++k) t[r] = t[r] + p[k][r];
           }
         }
+        return t;
+      };
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        g[i] = total(i, kg);
+        if constexpr (SW) u[i] = total(i, kg + 2);
       }
     }
     if (quant) lds_barrier();  // every read of the partial sums is done
@@ -361,6 +437,8 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
       for (int i = 0; i < MT; ++i) emit(i, kg, g[i], u[i]);
     }
   } else {
+    if (kept) add_saved();
+    if (quant) lds_barrier();  // every read of the saved sums is done
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -448,50 +526,54 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
     a.tm = (nb + bm - 1) / bm;
     return (t + 7) / 8 * 8 * a.tm;
   };
-  // Tile by the number of 32 x 32 output tiles (waves' worth of work; the chip
-  // holds 4096 waves at 4 per SIMD). Many: 64 activation rows per wave halve
+  // Tile by the number of 32 x 32 output tiles per CU (a tile is a wave's work; a
+  // CU holds 16 waves at 4 per SIMD). Many: 64 activation rows per wave halve
   // the decode per output, K unsplit. Fewer: 32 rows, and K split over the
-  // groups of a workgroup so that every SIMD has waves to overlap. Measured
-  // (us, tiles; the chosen one first): gate+up 5120 -> 2 x 17408, 512 rows
-  // (17408 tiles) 2,4,1 233, 1,4,1 259, 1,2,4 300; 128 rows (4352) 1,4,1 82,
-  // 2,4,1 84, 1,2,4 81; 64 rows (2176) 1,2,4 48, 1,4,1 51, 1,2,8 63; down
-  // 17408 -> 5120, 203 rows (1120) 1,2,4 93, 1,4,1 117, 1,2,8 103; 5120 ->
-  // 5120, 64 rows (320) 1,2,8 13.4, 1,2,4 14.0, 1,1,4 15.6; gate+up of 32 rows
-  // (1088) 1,2,4 34, 1,4,1 37, 1,2,8 41; 5120 -> 3 x 5120, 32 rows (480)
-  // 1,2,8 15.8, 1,2,4 16.2; 2048 -> 2 x 2048, 96 rows (384) 1,2,4 7.7, 1,2,8
-  // 8.7. At most one tile per CU: a workgroup of one tile, on as many CUs as
-  // there are tiles; 32 rows, 5120 -> 5120 (160) 1,1,8 9.7, 1,2,8 12.8, 1,1,4
-  // 11.4; down (160) 1,1,12 27.4, 1,1,8 28.8, 1,2,8 36; 4096 -> 2048 (64) 1,1,8
-  // 7.8, 1,1,12 8.1, 1,2,8 10.5; 1024 -> 1024 (32) 1,1,4 4.22, 1,1,8 4.22, 1,2,8
-  // 5.4; one block per group: 512 -> 3 x 4096, 64 rows (768) 1,1,4 5.0, 1,2,4 5.5.
-  // K unsplit from 3000 tiles: 3072 -> 3072, 1000 rows (3072) 1,4,1 37, 1,2,4 40;
-  // and from 1024 where a group would have at most one block: 256 -> 3 x 2048,
-  // 512 rows (3072) 1,4,1 7.2, 1,2,4 12.4.
-  // (qout does not change the K split: y is the same with and without it.)
+  // groups of a workgroup so that every SIMD has waves to overlap. The bits of y
+  // are the same in all of them. Measured on 256 CUs (us; tiles; the chosen one
+  // first):
+  //  - from 32 per CU: gate+up 5120 -> 2 x 17408, 512 rows (17408) 2,4,1 248,
+  //    1,4,1 273, 1,2,4 316; 256 rows (8704) 2,4,1 140, 1,4,1 146; 5120 -> 8192,
+  //    1024 rows (8192) 2,4,1 123, 1,4,1 138; below: gate+up, 224 rows (7616)
+  //    1,4,1 130, 2,4,1 139; 5120 -> 8192, 800 rows (6400) 1,4,1 116, 2,4,1 120;
+  //  - from 10 per CU K unsplit: 600 rows of 5120 -> 5120 (3040) 1,4,1 55.8, 1,2,4
+  //    60.0; 544 rows (2720) 54.0 / 57.9; 160 rows of 5120 -> 17408 (2720) 53.2 / 56.4;
+  //    3072 -> 5376, 512 rows (2688) 35.5 / 37.4; below: 5120 -> 5120, 512 rows (2560)
+  //    1,2,4 50.2, 1,4,1 52.9; gate+up, 64 rows (2176) 48.7 / 51.1; down 17408 ->
+  //    5120, 203 rows (1120) 94.7 / 118;
+  //  - from 4 per CU where a group would have one block at most: 256 -> 4096, 320
+  //    rows (1280) 1,4,1 5.3, 1,1,4 6.3, 1,2,4 7.5; 384 -> 4096, 512 rows (2048)
+  //    7.2 / 9.2 / 9.3; below: 512 -> 3 x 4096, 64 rows (768) 1,1,4 4.8, 1,2,4 5.6,
+  //    1,4,1 6.4;
+  //  - up to one per CU a workgroup of one tile, on as many CUs as there are tiles:
+  //    32 rows of 5120 -> 5120 (160) 1,1,8 9.5, 1,2,8 12.9; 4096 -> 8192 (256) 8.8 /
+  //    11.6; down (160) 28.4 / 35.6; 2048 -> 8192 (256) 1,1,4 6.0, 1,2,4 7.4; 1024 ->
+  //    1024 (32) 4.2 / 5.3;
+  //  - up to two per CU eight groups where K has eight shares: 5120 -> 3 x 5120, 32
+  //    rows (480) 1,2,8 14.7, 1,2,4 15.6; 8192 -> 8192, 64 rows (512) 20.5 / 21.2; 4096
+  //    -> 2 x 4096, 40 rows (512) 11.9 / 12.8; 3072 -> 6144, 64 rows (384) 9.5 / 9.9;
+  //    past that 2304 -> 9000, 64 rows (564) 1,2,4 12.1, 1,2,8 14.4; 5120 -> 5120, 128
+  //    rows (640) 21.7 / 24.9.
   const int per = mode == BTF_GEMV_SWIGLU ? 16 : 32;  // output rows of a wave
   tiles(per, 32);
   const int64_t t32 = (int64_t)a.tn * a.tm;
   if (t32 == 0) return BTF_OK;
-  if (t32 >= 8192 && nb > 32) {
+  const int64_t cus = 256;
+  bool eight = true;  // every matrix has eight shares of K
+  for (int i = 0; i < nuse; ++i) eight = eight && (segs[i].N == 0 || k_shares_log2(K / 128, segs[i].N) == 3);
+  const bool wide = qout && mode == BTF_GEMV_SWIGLU;  // (its Q8 blocks are two waves wide)
+  if (t32 >= 32 * cus && nb > 32) {
     by_mode<2, 4, 1>(mode, a, tiles(4 * per, 64), st);
-  } else if (t32 >= 3000 || (K <= 512 && t32 >= 1024)) {
+  } else if (t32 > 10 * cus || (K <= 512 && t32 >= 4 * cus)) {
     by_mode<1, 4, 1>(mode, a, tiles(4 * per, 32), st);
-  } else if (t32 <= 256 || (K <= 512 && t32 < 1024)) {
-    // (a swiglu's Q8 blocks are two waves wide: the same K split, so the same y)
-    const bool wide = qout && mode == BTF_GEMV_SWIGLU;
-    if (K <= 1024) {
-      if (wide) by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
-      else by_mode<1, 1, 4>(mode, a, tiles(per, 32), st);
-    } else if (K < 12288 || mode == BTF_GEMV_SWIGLU) {
-      if (wide) by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);
-      else by_mode<1, 1, 8>(mode, a, tiles(per, 32), st);
-    } else {
-      by_mode<1, 1, 12>(mode, a, tiles(per, 32), st);
-    }
-  } else if (t32 >= 500 || K < 4096) {
-    by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
-  } else {
+  } else if (eight && t32 <= cus && !wide) {
+    by_mode<1, 1, 8>(mode, a, tiles(per, 32), st);
+  } else if (eight && t32 <= 2 * cus) {
     by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);
+  } else if (K <= 2048 && (t32 <= cus || K <= 512) && !wide) {
+    by_mode<1, 1, 4>(mode, a, tiles(per, 32), st);
+  } else {
+    by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
   }
   return launch_status("gemm_t32_kernel");
 }

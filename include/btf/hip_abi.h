@@ -94,7 +94,11 @@ int btf_hip_launch_prep(const float* x, int ldx, int M, int n, const float* norm
 /* Replaces btf::cuda::launch_gemv (kernels.cuh:53-56). STORE / ADD:
  * y = W x or y += W x for each of the 1..3 segments (all share K and x).
  * SWIGLU: segs[0] = gate, segs[1] = up (same N); segs[0].y = silu(g) * u and
- * segs[1].y is unused. Requires K % 128 == 0. Any M >= 1. */
+ * segs[1].y is unused. Requires K % 128 == 0. Any M >= 1.
+ * More than 16 rows (on the int8-MFMA path): the order of an output's sums, and
+ * so its bits, follow from its matrix's K and N alone. They do not depend on M,
+ * on the row's place, on the other segments or on STORE / ADD / SWIGLU, so a
+ * prompt in pieces of more than 16 rows gives what it gives whole. */
 int btf_hip_launch_gemv(const btf_gemv_seg* segs, int nseg, int K, int M, const btf_q8act* a, int mode,
                         btf_stream_t stream);
 

@@ -1,9 +1,9 @@
 """The 32x32-tile GEMM (more than 16 activation rows) in each of its tile
-shapes, at the edges of tiles, segments and K groups.
+shapes, at the edges of tiles, segments and shares of K.
 
 Oracle: the exact int32 I of the oracle, scaled and summed in float64. An
 output is one rounding per sub-block product, at most four per 128-column
-block inside it, one per block of a group's chain and one per group, so
+block inside it, one per block of a share's chain and one per share, so
     |y - y64| <= (nblocks + 16) * 2^-24 * sum |scale * d * I|
 (each rounding is at most 2^-24 of a partial sum that the sum of magnitudes
 bounds); swiglu adds its own few roundings (2^-20 of the product's bound,
@@ -49,23 +49,27 @@ def wide(oracle, mat, sel, K, q, d, s):
     return t.sum(-1), np.abs(t).sum(-1)
 
 
-# (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses
+# (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses. K has four
+# shares up to 2048, eight past that.
 CASES = [
     (128, 17, [1, 33], 1),           # one activation tile with 15 dead rows, one block: three of four K groups have none
     (256, 32, [16070, 5], 8030),     # 504 / 502 tiles of few blocks: one wave x four groups, one full activation tile
     (128, 25, [131105], 65600),      # 4098 / 4100 tiles of one activation tile: four waves, K unsplit
     (384, 64, [37, 70, 9], 17),      # three blocks over four groups, three segments
-    (1152, 95, [45], 50),            # one wave x eight groups, nine blocks: uneven groups, a dead row in the last tile
+    (1152, 95, [45], 50),            # one wave x four groups, nine blocks: uneven groups, a dead row in the last tile
     (1152, 32, [8161], 4081),        # 256 / 256 tiles: the last of one tile per workgroup
     (1152, 32, [8193], 4097),        # 257 / 257 tiles: two waves x four groups
-    (12416, 40, [37, 5], 20),        # one wave x twelve groups (swiglu: eight), 97 blocks
+    (12416, 40, [37, 5], 20),        # one wave x eight groups, 97 blocks
     (4224, 64, [4200], 2200),        # 264 / 276 tiles: two waves x eight groups, 33 blocks
     (640, 65, [6917], 3500),         # 651 / 657 tiles: two waves x four groups; five blocks
     (640, 32, [16070, 5], 8030),     # the same of one full activation tile
+    (2176, 40, [16100, 20], 8100),   # 1008 / 1014 tiles: two waves x four groups of two shares, 17 blocks
     (512, 520, [2000], 1000),        # 1071 / 1071 tiles of few blocks: four waves, K unsplit
-    (1152, 1000, [3000], 1500),      # 3008 / 3008 tiles: four waves, K unsplit
+    (1152, 1000, [3000], 1500),      # 3008 / 3008 tiles: four waves, K unsplit, four shares
+    (2176, 900, [3000], 1500),       # 2726 / 2726 tiles: the same, eight shares of two or three blocks
     (256, 200, [18733], 9400),       # 4102 / 4116 tiles: four waves, K unsplit
     (256, 513, [15500], 7800),       # 8245 / 8296 tiles: 64 activation rows a wave, the last tile nearly empty
+    (2176, 513, [15500], 7800),      # the same, eight shares
 ]
 
 
@@ -181,3 +185,42 @@ def test_dot4_two_rows_equal_one_row_launches(hip, oracle, K, N):
     I = torch.zeros((2, N, K // 32), dtype=torch.int32, device="cuda")
     hip.gemv_i32_dump(w[0][0], N, K, 2, hip.Q8Act(dev(q), dev(d), dev(s)), I, stream())
     assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(mats[0][0], K, q, s))
+
+
+@pytest.mark.parametrize("K,wide_n", [(128, 9000), (640, 9000), (1152, 9000), (2176, 16390), (4224, 9000),
+                                      (12416, 9000)])
+def test_t32_rows_do_not_depend_on_the_launch(hip, K, wide_n):
+    """More than 16 rows: an output's bits are the same however many rows and
+    segments its launch has and in every tile shape that these choose, with
+    gate and up in a swiglu too. K of one block, and of block counts that its
+    shares do not divide; segments of four and of eight shares in one launch."""
+    torch = _torch()
+    G = hip.GemvMode
+    rng = np.random.default_rng(K)
+    M, N = 1000, 1030
+    q = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    d = (0.001 + rng.random((M, K // 32)) * 0.05).astype(np.float16).astype(np.float32)
+    s = q.reshape(M, K // 32, 32).sum(-1, dtype=np.int32)
+    a, b, c = ([dev(t) for t in matrix(rng, n, K)] for n in (N, wide_n, N))
+
+    def run(rows, mode, *mats):
+        act = hip.Q8Act(dev(q[rows]), dev(d[rows]), dev(s[rows]))
+        m = len(rows)
+        ys = [torch.zeros((m, w[0].shape[0]), device="cuda") for w in mats]
+        segs = [hip.GemvSeg(*w, w[0].shape[0], y, w[0].shape[0]) for w, y in zip(mats, ys)]
+        hip.launch_gemv(segs, K, m, act, mode, stream())
+        return [y.cpu().numpy().view(np.uint32) for y in ys]
+
+    every = np.arange(M)
+    ya, yb, yc = run(every, G.kStore, a, b, c)
+    sw = run(every, G.kSwiglu, a, c)[0]
+    for i, (y, w) in enumerate(((ya, a), (yb, b), (yc, c))):
+        assert np.array_equal(run(every, G.kStore, w)[0], y), f"matrix {i} alone"
+    # tiles of 32 x 32 outputs: 33 (a) and 315 (a and b of 9000) times a row group of 32
+    for n in (17, 32, 40, 95, 200, 400, 513):
+        rows = every[300:300 + n]
+        assert np.array_equal(run(rows, G.kStore, a)[0], ya[rows]), f"{n} rows, one segment"
+        got = run(rows, G.kStore, b, a)
+        assert np.array_equal(got[0], yb[rows]) and np.array_equal(got[1], ya[rows]), f"{n} rows, two segments"
+        assert np.array_equal(run(rows, G.kSwiglu, a, c)[0], sw[rows]), f"{n} rows, swiglu"
+        assert np.array_equal(run(rows, G.kAdd, a)[0], ya[rows]), f"{n} rows, added to zeros"
