@@ -124,6 +124,7 @@ _launch_gemv_ptq1_0 = _decl("btf_hip_launch_gemv_ptq1_0",
                             [C.POINTER(_GemvSeg), _i, _i, _i, C.POINTER(_Q8Act), _i, _vp])
 _dump = _decl("btf_hip_gemv_i32_dump", [_vp, _i, _i, _i, C.POINTER(_Q8Act), _vp, _vp])
 _set_policy = _decl("btf_hip_gemv_set_policy", [_i])
+_gemm_tile = _decl("btf_hip_gemm_tile", [_i, C.POINTER(_i), _i, _i, _i, _i, _i])
 _gen = _decl("btf_hip_gen_ptq1_0", [C.c_uint64, C.c_uint64, _i64, _i64, _vp, _vp])
 _stream_read = _decl("btf_hip_stream_read", [_vp, C.c_uint64, C.c_uint32, _vp, _vp])
 _last_error = _decl("btf_hip_last_error", [], C.c_char_p)
@@ -169,7 +170,7 @@ _loader_destroy = _decl("btf_hip_loader_destroy", [_vp])
 ABI_SYMBOLS = (
     "btf_hip_kernels_init", "btf_hip_gemv_max_nb", "btf_hip_launch_repack", "btf_hip_launch_prep",
     "btf_hip_launch_gemv", "btf_hip_launch_gemv_ex", "btf_hip_launch_gemv_ptq1_0", "btf_hip_launch_embed", "btf_hip_argmax_part_bytes",
-    "btf_hip_launch_argmax", "btf_hip_launch_argmax_noalloc", "btf_hip_launch_pos_add", "btf_hip_last_error", "btf_hip_gemv_i32_dump", "btf_hip_gemv_set_policy",
+    "btf_hip_launch_argmax", "btf_hip_launch_argmax_noalloc", "btf_hip_launch_pos_add", "btf_hip_last_error", "btf_hip_gemv_i32_dump", "btf_hip_gemv_set_policy", "btf_hip_gemm_tile",
     "btf_hip_gen_ptq1_0", "btf_hip_stream_read", "btf_hip_device_info", "btf_hip_device_count", "btf_hip_set_device", "btf_hip_malloc",
     "btf_hip_free", "btf_hip_host_alloc_mapped", "btf_hip_host_free", "btf_hip_memcpy_h2d", "btf_hip_memcpy_d2h",
     "btf_hip_memset", "btf_hip_device_synchronize", "btf_hip_stream_create", "btf_hip_stream_destroy",
@@ -415,6 +416,13 @@ def gemv_i32_dump(codes, N: int, K: int, M: int, a: Q8Act, I_out, stream=None) -
 def gemv_set_policy(mfma_min_m: int) -> int:
     """Batches of M >= mfma_min_m use the int8-MFMA kernel; 0 = default. Returns the previous value."""
     return _set_policy(mfma_min_m)
+
+
+def gemm_tile(cu_count: int, N, K: int, M: int, mode: GemvMode = GemvMode.kStore, q8_out: bool = False):
+    """(32-row activation tiles per wave, waves along the outputs, K groups) of
+    a launch of M > 16 rows on `cu_count` CUs, or None. N: the segments' outputs."""
+    t = _gemm_tile(cu_count, (C.c_int * len(N))(*N), len(N), K, M, int(mode), int(q8_out))
+    return (t // 10000, t // 100 % 100, t % 100) if t else None
 
 
 def gen_ptq1_0(seed: int, mat: int, first_block: int, nblocks: int, dst, stream=None) -> None:

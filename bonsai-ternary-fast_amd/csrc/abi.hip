@@ -315,6 +315,13 @@ int btf_hip_gemv_set_policy(int mfma_min_m) {
   return prev;
 }
 
+int btf_hip_gemm_tile(int cu_count, const int* N, int nseg, int K, int M, int mode, int q8_out) {
+  if (!N || nseg < 1 || nseg > 3 || K <= 0 || K % 128 || M <= 16 || cu_count <= 0) return 0;
+  int n[3] = {};
+  for (int i = 0; i < (mode == BTF_GEMV_SWIGLU ? 1 : nseg); ++i) n[i] = N[i];
+  return gemm_t32_tile(n, K, M, mode, q8_out != 0, cu_count);
+}
+
 int btf_hip_stream_read(const void* src, uint64_t bytes, uint32_t never, uint32_t* sink, btf_stream_t stream) {
   if (bytes == 0) return BTF_OK;
   if (!src || !sink || !aligned(src, 16) || bytes % 16)

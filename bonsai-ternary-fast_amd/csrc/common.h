@@ -170,7 +170,8 @@ int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& a,
               hipStream_t st, const DevState& ds, const Q8* qout = nullptr);
 // 32x32-tile MFMA path (more than 16 rows). qout: also the Q8 of the output rows (nb <= 32, N % 32 == 0).
 int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-             hipStream_t st, const Q8* qout = nullptr);
+             hipStream_t st, const DevState& ds, const Q8* qout = nullptr);
+int gemm_t32_tile(const int (&N)[3], int K, int nb, int mode, bool q8, int cus);  // 10000 MT + 100 WN + WK; 0: no outputs
 int mfma_rows_per_pass();
 
 int repack(const uint8_t* src, int64_t nblocks, uint8_t* codes, uint16_t* scales, hipStream_t st,

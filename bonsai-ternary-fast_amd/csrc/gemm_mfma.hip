@@ -754,10 +754,10 @@ void by_waves_kp(int nw, int mode, const MfmaArgs& a, dim3 grid, hipStream_t st)
 int mfma_rows_per_pass() { return 64; }
 
 int gemm_mfma(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-              hipStream_t st, const DevState&, const Q8* qout) {
+              hipStream_t st, const DevState& ds, const Q8* qout) {
   MfmaArgs a{};
   if (qout && nb > 32) return fail(BTF_ERR_ARGS, "gemm: a Q8 output needs at most 32 rows");
-  if (nb > 16) return gemm_t32(segs, nseg, K, m0, nb, act, mode, dump, st, qout);
+  if (nb > 16) return gemm_t32(segs, nseg, K, m0, nb, act, mode, dump, st, ds, qout);
   // the K-split 16-row tile (32 rows with a Q8 output)
   if (qout && dump) return fail(BTF_ERR_ARGS, "gemm: a Q8 output has no dump");
   const int rows_real = qout ? 32 : 16;

@@ -483,10 +483,68 @@ void by_mode(int mode, const T32Args& a, int grid, hipStream_t st) {  // (a by r
     hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, BTF_GEMV_SWIGLU, false>), dim3(grid), blk, 0, st, a);
 }
 
+// Output rows of a wave.
+constexpr int t32_rows(int mode) { return mode == BTF_GEMV_SWIGLU ? 16 : 32; }
+
+struct T32Tile {
+  int mt, wn, wk;  // mt 0: no outputs
+};
+
+// Tile by the number of 32 x 32 output tiles per CU (a tile is a wave's work; a
+// CU holds 16 waves at 4 per SIMD). Many: 64 activation rows per wave halve
+// the decode per output, K unsplit. Fewer: 32 rows, and K split over the
+// groups of a workgroup so that every SIMD has waves to overlap. The bits of y
+// are the same in all of them. Measured on 256 CUs (us; tiles; the chosen one
+// first):
+//  - from 32 per CU: gate+up 5120 -> 2 x 17408, 512 rows (17408) 2,4,1 248,
+//    1,4,1 273, 1,2,4 316; 256 rows (8704) 2,4,1 140, 1,4,1 146; 5120 -> 8192,
+//    1024 rows (8192) 2,4,1 123, 1,4,1 138; below: gate+up, 224 rows (7616)
+//    1,4,1 130, 2,4,1 139; 5120 -> 8192, 800 rows (6400) 1,4,1 116, 2,4,1 120;
+//  - from 10 per CU K unsplit: 600 rows of 5120 -> 5120 (3040) 1,4,1 55.8, 1,2,4
+//    60.0; 544 rows (2720) 54.0 / 57.9; 160 rows of 5120 -> 17408 (2720) 53.2 / 56.4;
+//    3072 -> 5376, 512 rows (2688) 35.5 / 37.4; below: 5120 -> 5120, 512 rows (2560)
+//    1,2,4 50.2, 1,4,1 52.9; gate+up, 64 rows (2176) 48.7 / 51.1; down 17408 ->
+//    5120, 203 rows (1120) 94.7 / 118;
+//  - from 4 per CU where a group would have one block at most: 256 -> 4096, 320
+//    rows (1280) 1,4,1 5.3, 1,1,4 6.3, 1,2,4 7.5; 384 -> 4096, 512 rows (2048)
+//    7.2 / 9.2 / 9.3; below: 512 -> 3 x 4096, 64 rows (768) 1,1,4 4.8, 1,2,4 5.6,
+//    1,4,1 6.4;
+//  - up to one per CU a workgroup of one tile, on as many CUs as there are tiles:
+//    32 rows of 5120 -> 5120 (160) 1,1,8 9.5, 1,2,8 12.9; 4096 -> 8192 (256) 8.8 /
+//    11.6; down (160) 28.4 / 35.6; 2048 -> 8192 (256) 1,1,4 6.0, 1,2,4 7.4; 1024 ->
+//    1024 (32) 4.2 / 5.3;
+//  - up to two per CU eight groups where K has eight shares: 5120 -> 3 x 5120, 32
+//    rows (480) 1,2,8 14.7, 1,2,4 15.6; 8192 -> 8192, 64 rows (512) 20.5 / 21.2; 4096
+//    -> 2 x 4096, 40 rows (512) 11.9 / 12.8; 3072 -> 6144, 64 rows (384) 9.5 / 9.9;
+//    past that 2304 -> 9000, 64 rows (564) 1,2,4 12.1, 1,2,8 14.4; 5120 -> 5120, 128
+//    rows (640) 21.7 / 24.9.
+T32Tile t32_tile(const int (&N)[3], int K, int nb, int mode, bool q8, int64_t cus) {
+  int64_t n = 0;
+  bool eight = true;  // every matrix has eight shares of K
+  for (int i = 0; i < 3; ++i) {
+    n += (N[i] + t32_rows(mode) - 1) / t32_rows(mode);
+    eight = eight && (N[i] == 0 || k_shares_log2(K / 128, N[i]) == 3);
+  }
+  const int64_t t32 = n * ((nb + 31) / 32);
+  const bool wide = q8 && mode == BTF_GEMV_SWIGLU;  // (its Q8 blocks are two waves wide)
+  if (t32 == 0) return {0, 0, 0};
+  if (t32 >= 32 * cus && nb > 32) return {2, 4, 1};
+  if (t32 > 10 * cus || (K <= 512 && t32 >= 4 * cus)) return {1, 4, 1};
+  if (eight && t32 <= cus && !wide) return {1, 1, 8};
+  if (eight && t32 <= 2 * cus) return {1, 2, 8};
+  if (K <= 2048 && (t32 <= cus || K <= 512) && !wide) return {1, 1, 4};
+  return {1, 2, 4};
+}
+
 }  // namespace
 
+int gemm_t32_tile(const int (&N)[3], int K, int nb, int mode, bool q8, int cus) {
+  const T32Tile t = t32_tile(N, K, nb, mode, q8, cus);
+  return 10000 * t.mt + 100 * t.wn + t.wk;
+}
+
 int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act, int mode, int32_t* dump,
-             hipStream_t st, const Q8* qout) {
+             hipStream_t st, const DevState& ds, const Q8* qout) {
   T32Args a{};
   const int nuse = mode == BTF_GEMV_SWIGLU ? 1 : nseg;
   a.K = K;
@@ -526,55 +584,22 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
     a.tm = (nb + bm - 1) / bm;
     return (t + 7) / 8 * 8 * a.tm;
   };
-  // Tile by the number of 32 x 32 output tiles per CU (a tile is a wave's work; a
-  // CU holds 16 waves at 4 per SIMD). Many: 64 activation rows per wave halve
-  // the decode per output, K unsplit. Fewer: 32 rows, and K split over the
-  // groups of a workgroup so that every SIMD has waves to overlap. The bits of y
-  // are the same in all of them. Measured on 256 CUs (us; tiles; the chosen one
-  // first):
-  //  - from 32 per CU: gate+up 5120 -> 2 x 17408, 512 rows (17408) 2,4,1 248,
-  //    1,4,1 273, 1,2,4 316; 256 rows (8704) 2,4,1 140, 1,4,1 146; 5120 -> 8192,
-  //    1024 rows (8192) 2,4,1 123, 1,4,1 138; below: gate+up, 224 rows (7616)
-  //    1,4,1 130, 2,4,1 139; 5120 -> 8192, 800 rows (6400) 1,4,1 116, 2,4,1 120;
-  //  - from 10 per CU K unsplit: 600 rows of 5120 -> 5120 (3040) 1,4,1 55.8, 1,2,4
-  //    60.0; 544 rows (2720) 54.0 / 57.9; 160 rows of 5120 -> 17408 (2720) 53.2 / 56.4;
-  //    3072 -> 5376, 512 rows (2688) 35.5 / 37.4; below: 5120 -> 5120, 512 rows (2560)
-  //    1,2,4 50.2, 1,4,1 52.9; gate+up, 64 rows (2176) 48.7 / 51.1; down 17408 ->
-  //    5120, 203 rows (1120) 94.7 / 118;
-  //  - from 4 per CU where a group would have one block at most: 256 -> 4096, 320
-  //    rows (1280) 1,4,1 5.3, 1,1,4 6.3, 1,2,4 7.5; 384 -> 4096, 512 rows (2048)
-  //    7.2 / 9.2 / 9.3; below: 512 -> 3 x 4096, 64 rows (768) 1,1,4 4.8, 1,2,4 5.6,
-  //    1,4,1 6.4;
-  //  - up to one per CU a workgroup of one tile, on as many CUs as there are tiles:
-  //    32 rows of 5120 -> 5120 (160) 1,1,8 9.5, 1,2,8 12.9; 4096 -> 8192 (256) 8.8 /
-  //    11.6; down (160) 28.4 / 35.6; 2048 -> 8192 (256) 1,1,4 6.0, 1,2,4 7.4; 1024 ->
-  //    1024 (32) 4.2 / 5.3;
-  //  - up to two per CU eight groups where K has eight shares: 5120 -> 3 x 5120, 32
-  //    rows (480) 1,2,8 14.7, 1,2,4 15.6; 8192 -> 8192, 64 rows (512) 20.5 / 21.2; 4096
-  //    -> 2 x 4096, 40 rows (512) 11.9 / 12.8; 3072 -> 6144, 64 rows (384) 9.5 / 9.9;
-  //    past that 2304 -> 9000, 64 rows (564) 1,2,4 12.1, 1,2,8 14.4; 5120 -> 5120, 128
-  //    rows (640) 21.7 / 24.9.
-  const int per = mode == BTF_GEMV_SWIGLU ? 16 : 32;  // output rows of a wave
-  tiles(per, 32);
-  const int64_t t32 = (int64_t)a.tn * a.tm;
-  if (t32 == 0) return BTF_OK;
-  const int64_t cus = 256;
-  bool eight = true;  // every matrix has eight shares of K
-  for (int i = 0; i < nuse; ++i) eight = eight && (segs[i].N == 0 || k_shares_log2(K / 128, segs[i].N) == 3);
-  const bool wide = qout && mode == BTF_GEMV_SWIGLU;  // (its Q8 blocks are two waves wide)
-  if (t32 >= 32 * cus && nb > 32) {
-    by_mode<2, 4, 1>(mode, a, tiles(4 * per, 64), st);
-  } else if (t32 > 10 * cus || (K <= 512 && t32 >= 4 * cus)) {
-    by_mode<1, 4, 1>(mode, a, tiles(4 * per, 32), st);
-  } else if (eight && t32 <= cus && !wide) {
-    by_mode<1, 1, 8>(mode, a, tiles(per, 32), st);
-  } else if (eight && t32 <= 2 * cus) {
-    by_mode<1, 2, 8>(mode, a, tiles(2 * per, 32), st);
-  } else if (K <= 2048 && (t32 <= cus || K <= 512) && !wide) {
-    by_mode<1, 1, 4>(mode, a, tiles(per, 32), st);
-  } else {
-    by_mode<1, 2, 4>(mode, a, tiles(2 * per, 32), st);
-  }
+  const int N[3] = {nuse > 0 ? segs[0].N : 0, nuse > 1 ? segs[1].N : 0, nuse > 2 ? segs[2].N : 0};
+  const T32Tile t = t32_tile(N, K, nb, mode, qout != nullptr, ds.cu_count);
+  if (t.mt == 0) return BTF_OK;
+  const int grid = tiles(t.wn * t32_rows(mode), 32 * t.mt);
+  if (t.mt == 2)
+    by_mode<2, 4, 1>(mode, a, grid, st);
+  else if (t.wn == 4)
+    by_mode<1, 4, 1>(mode, a, grid, st);
+  else if (t.wn == 2 && t.wk == 8)
+    by_mode<1, 2, 8>(mode, a, grid, st);
+  else if (t.wn == 2)
+    by_mode<1, 2, 4>(mode, a, grid, st);
+  else if (t.wk == 8)
+    by_mode<1, 1, 8>(mode, a, grid, st);
+  else
+    by_mode<1, 1, 4>(mode, a, grid, st);
   return launch_status("gemm_t32_kernel");
 }
 

@@ -186,6 +186,12 @@ int btf_hip_launch_gemv_ptq1_0(const btf_gemv_seg* segs, int nseg, int K, int M,
  * Process-global; for tests and benchmarks. Returns the previous value. */
 int btf_hip_gemv_set_policy(int mfma_min_m);
 
+/* Test hook, host only: the tile that a launch of M > 16 rows takes on a GPU of
+ * `cu_count` CUs, as 10000 * (32-row activation tiles per wave) + 100 * (waves
+ * along the outputs) + (groups that split K); 0 for no outputs or M <= 16. N: the
+ * outputs of the nseg matrices; q8_out: with launch_gemv_ex's Q8 output. */
+int btf_hip_gemm_tile(int cu_count, const int* N, int nseg, int K, int M, int mode, int q8_out);
+
 /* Measurement hook, no reference counterpart: a plain streaming read of
  * `bytes` of device memory at src (16-byte words, non-temporal loads as the
  * GEMV kernels read their weights), the practical HBM read ceiling the GEMV
