@@ -27,8 +27,9 @@ def _flags():
     m = re.search(r"^HIPFLAGS\s*:=\s*(.*)$", text, re.M)
     flags = m.group(1).replace("$(ARCH)", "gfx950").split()
     per_file = {}
-    for f, extra in re.findall(r"^_build/(\w+)\.o:\s*HIPFLAGS\s*\+=\s*(.*)$", text, re.M):
-        per_file[f] = extra.split()
+    for targets, extra in re.findall(r"^([^#\n:]*):\s*HIPFLAGS\s*\+=\s*(.*)$", text, re.M):
+        for f in targets.split():
+            per_file.setdefault(re.fullmatch(r"_build/(\w+)\.o", f).group(1), []).extend(extra.split())
     return flags, per_file
 
 
@@ -58,6 +59,22 @@ def _remarks(src):
         elif cur is not None:
             cur[key] = int(val)
     return kernels
+
+
+def test_flags_are_those_of_the_build():
+    """The flags that the checks below compile with are the ones that make
+    passes for each source."""
+    flags, per_file = _flags()
+    out = subprocess.run(["make", "-n", "-B", "-C", PKG, "libbtf_hip.so", "HIPCC=hipcc", "ARCH=gfx950"],
+                         capture_output=True, text=True, check=True).stdout
+    built = {}
+    for line in out.splitlines():
+        m = re.match(r"hipcc (.*) -c (csrc/\w+\.hip) -o ", line.strip())
+        if m:
+            built[m.group(2)] = m.group(1).split()
+    assert sorted(built) == sorted(_sources())
+    for src, used in built.items():
+        assert flags + per_file.get(os.path.splitext(os.path.basename(src))[0], []) == used, src
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
