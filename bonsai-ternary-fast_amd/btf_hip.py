@@ -10,12 +10,14 @@ stream. Failures raise RuntimeError with the library's message, as the
 reference launchers throw std::runtime_error.
 
 There is no fallback: importing this module fails loudly when the HIP
-library has not been built.
+library has not been built. (The native launch calls of csrc/pycall.c are
+optional: without them the same library is called through ctypes.)
 """
 from __future__ import annotations
 
 import ctypes as C
 import enum
+import importlib.machinery
 import importlib.util
 import os
 import sys
@@ -23,16 +25,22 @@ from dataclasses import dataclass
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libbtf_hip.so")
-CALL_PATH = os.path.join(HERE, "_btf_call.so")
+# the native launch calls, if they were built for this Python (the suffix says for which)
+CALL_PATH = os.path.join(HERE, "_btf_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
-for _p in (LIB_PATH, CALL_PATH):
-    if not os.path.exists(_p):
-        raise ImportError(f"{_p} is missing: build it with `make -C {HERE}` (hipcc, gfx950)")
+if not os.path.exists(LIB_PATH):
+    raise ImportError(f"{LIB_PATH} is missing: build it with `make -C {HERE}` (hipcc, gfx950)")
 
 _lib = C.CDLL(LIB_PATH)
-_spec = importlib.util.spec_from_file_location("_btf_call", CALL_PATH)
-_call = importlib.util.module_from_spec(_spec)
-_spec.loader.exec_module(_call)
+if os.path.exists(CALL_PATH):
+    _spec = importlib.util.spec_from_file_location("_btf_call", CALL_PATH)
+    _call = importlib.util.module_from_spec(_spec)
+    _spec.loader.exec_module(_call)
+else:
+    class _call:
+        """No native calls: every launch takes the ctypes path."""
+        prep = gemv = gemv_ptq1_0 = gemv_ex = staticmethod(lambda *args: NotImplemented)
+        bind = staticmethod(lambda *args: None)
 
 BTF_OK, BTF_ERR_ARGS, BTF_ERR_DEVICE, BTF_ERR_LAUNCH, BTF_ERR_NOT_INIT = 0, 1, 2, 3, 4
 

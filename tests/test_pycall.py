@@ -3,6 +3,10 @@ same arguments as its ctypes path, over the forms that they read; every other
 form is left to the ctypes path. Host only: the calls are bound to recording
 callbacks instead of the launchers."""
 import ctypes as C
+import os
+import shutil
+import subprocess
+import sys
 import types
 
 import numpy as np
@@ -11,6 +15,7 @@ import torch
 
 import btf_hip as hip
 
+native = pytest.mark.skipif(not os.path.exists(hip.CALL_PATH), reason="native launch calls not built")
 vp = C.c_void_p
 Q8P, HXP, SEGP = C.POINTER(hip._Q8Act), C.POINTER(hip._Hx), C.POINTER(hip._GemvSeg)
 ARGS = {"prep": [vp, C.c_int, C.c_int, C.c_int, vp, C.c_float, HXP, vp, C.c_int, Q8P, vp],
@@ -52,6 +57,7 @@ ACTS = [hip.Q8Act(T[0], T[1], T[2]), hip.Q8Act(16, None, T[2]), hip.Q8Act()]
 STREAMS = [None, 0, 1 << 45, types.SimpleNamespace(cuda_stream=77)]
 
 
+@native
 @pytest.mark.parametrize("stream", STREAMS, ids=str)
 @pytest.mark.parametrize("a", ACTS, ids=["tensors", "mixed", "empty"])
 @pytest.mark.parametrize("hx", [None, hip.Hx(), hip.Hx(1024, 32, 2, 4, T[5]), hip.Hx(block=64, signs=4096)],
@@ -65,6 +71,7 @@ def test_prep_arguments(seen, stream, a, hx):
                  plain(a._c(), 0), hip._stream(stream) or None]
 
 
+@native
 @pytest.mark.parametrize("stream", STREAMS, ids=str)
 @pytest.mark.parametrize("nseg", [1, 2, 3])
 @pytest.mark.parametrize("kind", [list, tuple])
@@ -109,3 +116,39 @@ def test_errors_raise_the_library_message():
         hip.launch_gemv([hip.GemvSeg(T[0], T[1], 5, T[2], 7)], 100, 1, ACTS[0])
     with pytest.raises(RuntimeError, match="multiple of 32"):
         hip.launch_prep(T[3], 33, 1, 33, None, 0.0, None, None, 0, ACTS[0])
+
+
+def test_bindings_work_without_the_native_calls(tmp_path):
+    """A tree with the library alone imports, and its launches take the ctypes
+    path; native calls built for another Python are not loaded."""
+    shutil.copy(os.path.join(hip.HERE, "btf_hip.py"), tmp_path)
+    os.symlink(hip.LIB_PATH, tmp_path / "libbtf_hip.so")
+    for name in ("_btf_call.so", "_btf_call.cpython-39-x86_64-linux-gnu.so"):
+        (tmp_path / name).write_bytes(b"not for this Python")
+    code = """
+import btf_hip as h
+for f in (lambda: h.launch_prep(16, 33, 1, 33, None, 0.0, None, None, 0, h.Q8Act(16, 16, 16)),
+          lambda: h.launch_gemv([h.GemvSeg(16, 16, 5, 16, 5)], 100, 1, h.Q8Act(16, 16, 16)),
+          lambda: h.launch_gemv_ptq1_0([h.GemvSeg(16, None, 5, 16, 5)], 100, 1, h.Q8Act(16, 16, 16)),
+          lambda: h.launch_gemv_ex([h.GemvSeg(16, 16, 5, 16, 5)], 100, 1, h.Q8Act(16, 16, 16))):
+    try:
+        f()
+    except RuntimeError as e:
+        print(e)
+"""
+    out = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.count("multiple of") == 4, out.stdout
+
+
+def test_library_builds_without_python():
+    """`make` needs neither a Python nor its headers for the library itself."""
+    def targets(*args):
+        out = subprocess.run(["make", "-n", "-B", "-C", hip.HERE, "all", *args], capture_output=True, text=True)
+        assert out.returncode == 0, out.stderr
+        return out.stdout
+    assert "pycall.c" not in targets("PYTHON=/nonexistent/python3")
+    assert "pycall.c" not in targets("CC=/nonexistent/cc")
+    assert "libbtf_hip.so" in targets("PYTHON=/nonexistent/python3")
+    if os.path.exists(hip.CALL_PATH):
+        assert os.path.basename(hip.CALL_PATH) in targets(f"PYTHON={sys.executable}")
