@@ -3,6 +3,7 @@ Host only."""
 import random
 
 import pytest
+import torch  # noqa: F401  (before the library, so that the process has one HIP runtime: torch's)
 
 import btf_hip as hip
 
