@@ -129,13 +129,36 @@ def test_t32_modes_and_edges(hip, oracle, K, M, Ns, N2):
     assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(np.ascontiguousarray(mats[-1][0][:n]), K, q, s))
 
 
+# one launch for each tile: (tile, K, M, N)
+DUMPS = [((1, 1, 4), 128, 17, 45), ((1, 1, 8), 2176, 40, 45), ((1, 2, 8), 2176, 64, 4200), ((1, 2, 4), 640, 40, 8205),
+         ((1, 4, 1), 128, 513, 2005), ((2, 4, 1), 128, 513, 15500)]
+
+
+@pytest.mark.parametrize("tile,K,M,N", DUMPS)
+def test_t32_exact_dump_in_each_tile(hip, oracle, tile, K, M, N):
+    """The exact I, written by the tile that a launch of that size takes."""
+    torch = _torch()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert cus != 256 or hip.gemm_tile(cus, [N], K, M) == tile
+    rng = np.random.default_rng(K + M + N)
+    q, d, s = oracle.quantize_rows((rng.standard_normal((M, K)) * 2).astype(np.float32))
+    codes, _ = matrix(rng, N, K)
+    I = torch.full((M, N, K // 32), -(1 << 30), dtype=torch.int32, device="cuda")
+    hip.gemv_i32_dump(dev(codes), N, K, M, hip.Q8Act(dev(q), dev(d), dev(s)), I, stream())
+    assert int(I.min()) > -(1 << 30), "outputs not written"
+    sel = np.unique(np.r_[0:40, N // 2 - 20:N // 2 + 20, N - 40:N])
+    got = I[:, torch.from_numpy(sel).cuda()].cpu().numpy()
+    assert np.array_equal(got, oracle.gemv_i32(np.ascontiguousarray(codes[sel]), K, q, s))
+
+
 @pytest.mark.parametrize("K,M,N", [(128, 17, 64), (1152, 24, 96), (12416, 20, 64), (4224, 20, 8480),
                                    (1152, 32, 8224), (256, 32, 16064), (128, 30, 131136),
-                                   (128, 18, 262176)])
+                                   (128, 18, 262176), (256, 20, 32800)])
 def test_t32_q8_output(hip, oracle, K, M, N):
     """launch_gemv_ex with a Q8 output in each tile shape of one activation
     tile: y equals launch_gemv's bit for bit, the Q8 rows equal the oracle's
-    quantize of that y; the first block is all zero."""
+    quantize of that y; the first block is all zero. y starts from values of
+    its own, so that the add counts."""
     torch = _torch()
     rng = np.random.default_rng(K + M + N)
     q, d, s = oracle.quantize_rows((rng.standard_normal((M, K)) * 2).astype(np.float32))
@@ -143,12 +166,15 @@ def test_t32_q8_output(hip, oracle, K, M, N):
     mats = [matrix(rng, N, K) for _ in range(2)]
     mats[0][0][:32] = 0x55  # trit 0
     w = [(dev(c), dev(sc)) for c, sc in mats]
+    y0 = (rng.standard_normal((M, N)) * 8).astype(np.float32)
+    y0[:, :32] = 0
+    stored = None
     for mode in (hip.GemvMode.kStore, hip.GemvMode.kAdd, hip.GemvMode.kSwiglu):
         ys = []
         out = hip.Q8Act(torch.zeros((M, N), dtype=torch.int8, device="cuda"), torch.zeros((M, N // 32), device="cuda"),
                         torch.zeros((M, N // 32), dtype=torch.int32, device="cuda"))
         for fused in (False, True):
-            y = torch.zeros((M, N), device="cuda")
+            y = dev(y0)
             segs = [hip.GemvSeg(*w[0], N, y, N)] + ([hip.GemvSeg(*w[1], N, None, 0)] if mode == 2 else [])
             if fused:
                 hip.launch_gemv_ex(segs, K, M, act, mode=mode, out=out, stream=stream())
@@ -156,6 +182,10 @@ def test_t32_q8_output(hip, oracle, K, M, N):
                 hip.launch_gemv(segs, K, M, act, mode, stream())
             ys.append(y.cpu().numpy())
         assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32)), f"y, mode {mode}"
+        if mode == hip.GemvMode.kStore:
+            stored = ys[1]
+        elif mode == hip.GemvMode.kAdd:  # (more than 16 rows: the same sums as the store's)
+            assert np.array_equal(ys[1], y0 + stored), "the old y is not in the sum"
         rq, rd, rs = oracle.quantize_rows(ys[1])
         assert np.array_equal(out.q.cpu().numpy(), rq), f"q, mode {mode}"
         assert np.array_equal(out.d.cpu().numpy().view(np.uint32), rd.view(np.uint32)), f"d, mode {mode}"
