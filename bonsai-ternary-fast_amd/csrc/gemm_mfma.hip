@@ -99,8 +99,7 @@ __device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
 // arithmetic. The per-output sums do not depend on TR.
 template <int NW, int KB, int MODE, bool DUMP, int TR = 1>
 __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
-  constexpr int MT = 1;  // 16-row activation tiles
-  constexpr int BM = 16 * MT;
+  constexpr int BM = 16;  // activation rows
   constexpr int G1 = MODE == BTF_GEMV_SWIGLU ? 2 : 1;  // 16-row groups of a tile: gate (and up)
   constexpr int G = G1 * TR;                           // 16-row groups: tile t, matrix g1 at t * G1 + g1
   constexpr int RW = 16 * G;                           // staged rows per wave
@@ -141,13 +140,11 @@ __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
   const int kw0 = nsc * w / NW, kw1 = nsc * (w + 1) / NW;
   const int niter = ((nsc + NW - 1) / NW + KB - 1) / KB;
 
-  float acc[G][MT][4], blk[G][MT][4];
+  float acc[G][4], blk[G][4];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[g][mt][r] = 0.f;
+    for (int r = 0; r < 4; ++r) acc[g][r] = 0.f;
 
   u32x4 rc[NCV], rq[NQV];
   uint16_t rsc[NSV];
@@ -254,27 +251,24 @@ __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
           const uint32_t hi = __builtin_amdgcn_perm(0u, 0x000100FFu, (word >> (sh + 2)) & 0x03030303u);
           bfrag[g] = (long)(((uint64_t)hi << 32) | lo);
         }
+        const uint32_t* ap = &qsm[w][li * QS + 8 * sbx + 2 * t];
+        const long afrag = (long)(((uint64_t)ap[1] << 32) | ap[0]);
+        const v4i cin = {0, 0, 0, 0};
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const uint32_t* ap = &qsm[w][(16 * mt + li) * QS + 8 * sbx + 2 * t];
-          const long afrag = (long)(((uint64_t)ap[1] << 32) | ap[0]);
-          const v4i cin = {0, 0, 0, 0};
+        for (int g = 0; g < G; ++g) {
+          const v4i I = __builtin_amdgcn_mfma_i32_16x16x32_i8(afrag, bfrag[g], cin, 0, 0, 0);
+          if constexpr (DUMP) {
+            const int n = n0 + 16 * (g / G1) + li;
 #pragma unroll
-          for (int g = 0; g < G; ++g) {
-            const v4i I = __builtin_amdgcn_mfma_i32_16x16x32_i8(afrag, bfrag[g], cin, 0, 0, 0);
-            if constexpr (DUMP) {
-              const int n = n0 + 16 * (g / G1) + li;
+            for (int r = 0; r < 4; ++r) {
+              const int m = mb + 4 * t + r;
+              if (g % G1 == 0 && m < a.nb && n < N) a.dump[((size_t)(a.m0 + m) * N + n) * nsub + kb * 4 + sb] = I[r];
+            }
+          } else {
 #pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const int m = mb + 16 * mt + 4 * t + r;
-                if (g % G1 == 0 && m < a.nb && n < N) a.dump[((size_t)(a.m0 + m) * N + n) * nsub + kb * 4 + sb] = I[r];
-              }
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const float dv = dsm[w][sbx][16 * mt + 4 * t + r];
-                blk[g][mt][r] = sb == 0 ? dv * (float)I[r] : fmaf(dv, (float)I[r], blk[g][mt][r]);
-              }
+            for (int r = 0; r < 4; ++r) {
+              const float dv = dsm[w][sbx][4 * t + r];
+              blk[g][r] = sb == 0 ? dv * (float)I[r] : fmaf(dv, (float)I[r], blk[g][r]);
             }
           }
         }
@@ -284,9 +278,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
         for (int g = 0; g < G; ++g) {
           const float sc = h2f(scs[w][(16 * g + li) * KB + kbi]);
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[g][mt][r] = fmaf(sc, blk[g][mt][r], acc[g][mt][r]);
+          for (int r = 0; r < 4; ++r) acc[g][r] = fmaf(sc, blk[g][r], acc[g][r]);
         }
       }
     }  // kbi
@@ -299,9 +291,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_ks_kernel(MfmaArgs a) {
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[((w * G + g) * 16 + li) * BM + 16 * mt + 4 * t + r] = acc[g][mt][r];
+    for (int r = 0; r < 4; ++r) red[((w * G + g) * 16 + li) * BM + 4 * t + r] = acc[g][r];
   __syncthreads();
   // thread idx: output row rr = idx % RT of the tile, activation row mm = idx / RT
   // (with TR = 2 a half-wave holds the 32 outputs of one activation row: one Q8 block)

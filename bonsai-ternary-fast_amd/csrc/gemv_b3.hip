@@ -11,11 +11,16 @@
 // consecutive bytes j..j+3 are four consecutive elements, and their dot4
 // operand is one activation word as stored.
 //
-// Decode (two bytes per 16-bit lane): t = q*3 puts the
-// digit in each lane's high byte and the next q in its low byte; one
-// v_perm_b32 gathers the high bytes of the two lanes of two words (bytes
-// j, j+2 and j+1, j+3) into the dot4 operand of bytes j..j+3. Per 4 weights:
-// 2 multiplies, 1 permute, 1 dot4, 2 masks.
+// Decode: two bytes b of a word, one per 16-bit lane, times 3^n in one 24-bit
+// multiply; one v_perm_b32 gathers the high bytes H(n) of the two words of four
+// bytes j..j+3 into a dot4 operand, and the digits are H(n+1) - 3 H(n) (see Acc
+// below). Per 4 weights: 2 multiplies, 1 permute, about 2 dot4.
+//
+// What bounds it: neither the memory nor the vector ALU alone. At gate+up
+// (5120 -> 2 x 17408, one row, 15.3 us) the vector ALU is active 59 % of the time,
+// with 2.5 waves per SIMD on average that wait for 28 % of their cycles (SQ
+// counters). Its 1088 workgroups are 64 more than the 1024 that the chip holds at
+// 88 registers and five waves each, so a few run in a second round.
 //
 // Work decomposition: one lane owns one 128-weight block of a row; an
 // 8-lane group owns one 1024-column slice; a workgroup covers R rows per

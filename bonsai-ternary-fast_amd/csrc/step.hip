@@ -401,7 +401,7 @@ __device__ __forceinline__ bool early_finish(const OpDev& op, int lid, uint32_t 
 // writes the slice's Q8 into the LDS image, where the plain fetch would have
 // copied the producer's Q8 words. Bit-identical to launch_prep on the same
 // fp32 vector: the same per-slice arithmetic, and the RMSNorm scale from the
-// producers' block sums of squares summed in prep_slices_kernel's order.
+// producers' block sums of squares summed in prep_quad_kernel's order.
 struct PrepRegs {  // an op's prep fields in scalar registers
   const float* normw;
   const float* signs;
