@@ -93,7 +93,8 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int MT, int WN, int WK, int MODE, bool DUMP>
+// MS: the most shares of K that a group holds (1: exactly one, so nothing is set aside).
+template <int MT, int WN, int WK, int MS, int MODE, bool DUMP>
 __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_t32_kernel(T32Args a) {
   constexpr bool SW = MODE == BTF_GEMV_SWIGLU;
   constexpr int BM = 32 * MT;               // activation rows
@@ -107,9 +108,8 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
   constexpr int DB = BM * 4 * 4;            // d of a block: [sub-block][row]
   constexpr int SB = WN * 128;              // weight scales of a block: [staged row]
   constexpr int BUF = FB + DB + SB;
-  constexpr int MS = WK == 1 ? 8 : WN == 2 ? 8 / WK : 1;  // the most shares of K that a group holds
   constexpr int PART = WN * MT * 4096;      // a group's sums: [tile, chunk][thread]
-  constexpr int SAVE = MS > 1 && !DUMP ? PART : 0;  // those of the shares before its last one
+  constexpr int SAVE = MS > 1 ? PART : 0;  // those of the shares before its last one
   constexpr int GRP = 2 * BUF + SAVE;       // LDS of a group
   constexpr int OUT = MT == 1 ? 32 * (BNR + 1) * 4 : 0;  // outputs to quantize: [activation row][output]
   constexpr int LDS = WK * GRP > OUT ? WK * GRP : OUT;
@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (MS > 1 && !DUMP) {
+      if constexpr (MS > 1) {
         if (kb + 1 == kend && kend < k1) {  // the share ends here, and the group has another one
           if (WK == 1 && kept) add_saved();  // (a group that holds all of K adds its shares as it goes)
 #pragma unroll
@@ -470,17 +470,17 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
   }
 }
 
-template <int MT, int WN, int WK>
+template <int MT, int WN, int WK, int MS>
 void by_mode(int mode, const T32Args& a, int grid, hipStream_t st) {  // (a by reference: the grid's computation sets it)
   const dim3 blk(64 * WN * WK);
   if (a.dump)
-    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, BTF_GEMV_STORE, true>), dim3(grid), blk, 0, st, a);
+    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, 1, BTF_GEMV_STORE, true>), dim3(grid), blk, 0, st, a);
   else if (mode == BTF_GEMV_STORE)
-    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, BTF_GEMV_STORE, false>), dim3(grid), blk, 0, st, a);
+    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, MS, BTF_GEMV_STORE, false>), dim3(grid), blk, 0, st, a);
   else if (mode == BTF_GEMV_ADD)
-    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, BTF_GEMV_ADD, false>), dim3(grid), blk, 0, st, a);
+    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, MS, BTF_GEMV_ADD, false>), dim3(grid), blk, 0, st, a);
   else
-    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, BTF_GEMV_SWIGLU, false>), dim3(grid), blk, 0, st, a);
+    hipLaunchKernelGGL((gemm_t32_kernel<MT, WN, WK, MS, BTF_GEMV_SWIGLU, false>), dim3(grid), blk, 0, st, a);
 }
 
 // Output rows of a wave.
@@ -588,18 +588,22 @@ int gemm_t32(const GemvSeg* segs, int nseg, int K, int m0, int nb, const Q8& act
   const T32Tile t = t32_tile(N, K, nb, mode, qout != nullptr, ds.cu_count);
   if (t.mt == 0) return BTF_OK;
   const int grid = tiles(t.wn * t32_rows(mode), 32 * t.mt);
+  bool four = true;  // every matrix has four shares of K: one for each of four groups
+  for (int i = 0; i < nuse; ++i) four = four && (N[i] == 0 || k_shares_log2(K / 128, N[i]) == 2);
   if (t.mt == 2)
-    by_mode<2, 4, 1>(mode, a, grid, st);
+    by_mode<2, 4, 1, 8>(mode, a, grid, st);
   else if (t.wn == 4)
-    by_mode<1, 4, 1>(mode, a, grid, st);
+    by_mode<1, 4, 1, 8>(mode, a, grid, st);
   else if (t.wn == 2 && t.wk == 8)
-    by_mode<1, 2, 8>(mode, a, grid, st);
+    by_mode<1, 2, 8, 1>(mode, a, grid, st);
+  else if (t.wn == 2 && four)  // (1152 -> 16000, 32 rows: 5.98 us, 6.25 with the instance that sets sums aside)
+    by_mode<1, 2, 4, 1>(mode, a, grid, st);
   else if (t.wn == 2)
-    by_mode<1, 2, 4>(mode, a, grid, st);
+    by_mode<1, 2, 4, 2>(mode, a, grid, st);
   else if (t.wk == 8)
-    by_mode<1, 1, 8>(mode, a, grid, st);
+    by_mode<1, 1, 8, 1>(mode, a, grid, st);
   else
-    by_mode<1, 1, 4>(mode, a, grid, st);
+    by_mode<1, 1, 4, 1>(mode, a, grid, st);
   return launch_status("gemm_t32_kernel");
 }
 
