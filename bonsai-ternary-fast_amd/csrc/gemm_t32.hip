@@ -56,13 +56,15 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // y rows
 // every tile shape keeps to it, so an output of more than 16 rows has the same
 // bits whatever the launch's rows, segments and mode are. A tile that splits K
 // over fewer groups than G sets the sums of each share aside in LDS.
-// G is 8 where a launch of few rows splits K over 8 groups of waves (32 rows,
-// us, 4 groups / 8: 3072 -> 3072 7.5 / 6.6, 5120 -> 5120 11.2 / 9.5), and 4 where
-// that gains little (2048 -> 2048 5.9 / 5.6) or nothing (16384 outputs and more
-// fill the chip by themselves), because a tile that does not split K pays for each
-// share: gate+up of 512 rows (5120 -> 2 x 17408) 238 us with all of K in one
-// sum, 244 in 4 shares, 249 in 8; 2048 -> 2 x 8192, 512 rows, 49.5, 52.6, 55.3.
-__host__ __device__ constexpr int k_shares_log2(int nsc, int N) { return nsc <= 16 || N >= 16384 ? 2 : 3; }
+// G is 8 from K = 4096, where a launch of few rows splits K over 8 groups of waves
+// (32 rows of 5120 -> 5120: 9.5 us, over 4 groups 11.2; 3072 -> 3072 6.6 / 7.5). 4
+// below: eight chains of fewer than four blocks and their adds are further off 64
+// bits than four (2304 -> 6000: 6.4e-8 against 5.9e-8; even at 4096). And 4 for
+// 16384 outputs and more, which fill the chip by themselves: a tile that does not
+// split K pays for each share (gate+up of 512 rows, 5120 -> 2 x 17408: 238 us with
+// all of K in one sum, 244 in 4 shares, 249 in 8; 2048 -> 2 x 8192, 512 rows, 49.5,
+// 52.6, 55.3).
+__host__ __device__ constexpr int k_shares_log2(int nsc, int N) { return nsc < 32 || N >= 16384 ? 2 : 3; }
 
 struct T32Args {
   const uint8_t* codes[3];
@@ -405,7 +407,7 @@ __global__ void __launch_bounds__(64 * WN * WK, MT == 1 && WN > 1 ? 4 : 3) gemm_
         f32x4 p[WK], t;
 #pragma unroll
         for (int k = 0; k < WK; ++k) p[k] = partial(k, i, c);
-        if (kept) {  // two shares a group (of 17 blocks and more: none is empty)
+        if (kept) {  // two shares a group (of 32 blocks and more: none is empty)
           f32x4 v[WK];
 #pragma unroll
           for (int k = 0; k < WK; ++k) v[k] = saved(k, i, c);
@@ -515,9 +517,8 @@ struct T32Tile {
 //    1024 (32) 4.2 / 5.3;
 //  - up to two per CU eight groups where K has eight shares: 5120 -> 3 x 5120, 32
 //    rows (480) 1,2,8 14.7, 1,2,4 15.6; 8192 -> 8192, 64 rows (512) 20.5 / 21.2; 4096
-//    -> 2 x 4096, 40 rows (512) 11.9 / 12.8; 3072 -> 6144, 64 rows (384) 9.5 / 9.9;
-//    past that 2304 -> 9000, 64 rows (564) 1,2,4 12.1, 1,2,8 14.4; 5120 -> 5120, 128
-//    rows (640) 21.7 / 24.9.
+//    -> 2 x 4096, 40 rows (512) 11.9 / 12.8; past that 5120 -> 5120, 128 rows (640)
+//    1,2,4 21.7, 1,2,8 24.9; 17408 -> 5120, 128 rows (640) 59.6 / 71.6.
 T32Tile t32_tile(const int (&N)[3], int K, int nb, int mode, bool q8, int64_t cus) {
   int64_t n = 0;
   bool eight = true;  // every matrix has eight shares of K
@@ -532,7 +533,7 @@ T32Tile t32_tile(const int (&N)[3], int K, int nb, int mode, bool q8, int64_t cu
   if (t32 > 10 * cus || (K <= 512 && t32 >= 4 * cus)) return {1, 4, 1};
   if (eight && t32 <= cus && !wide) return {1, 1, 8};
   if (eight && t32 <= 2 * cus) return {1, 2, 8};
-  if (K <= 2048 && (t32 <= cus || K <= 512) && !wide) return {1, 1, 4};
+  if (K < 4096 && (t32 <= cus || K <= 512) && !wide) return {1, 1, 4};
   return {1, 2, 4};
 }
 

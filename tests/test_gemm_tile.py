@@ -14,7 +14,7 @@ TILES = {(2, 4, 1), (1, 4, 1), (1, 2, 4), (1, 2, 8), (1, 1, 4), (1, 1, 8)}
 
 def shares(K, N):
     """Shares of K in which a matrix's outputs are summed."""
-    return 4 if K <= 2048 or N >= 16384 else 8
+    return 4 if K < 4096 or N >= 16384 else 8
 
 
 @pytest.mark.parametrize("cus", CUS)
@@ -26,7 +26,7 @@ def test_every_choice_keeps_the_order_of_the_sums(cus):
     seen = set()
     for _ in range(20000):
         mode = rng.choice(list(hip.GemvMode))
-        K = 128 * rng.choice([1, 2, 4, 5, 8, 16, 17, 40, 97, 136, rng.randint(1, 300)])
+        K = 128 * rng.choice([1, 2, 4, 5, 8, 16, 31, 32, 40, 97, 136, rng.randint(1, 300)])
         N = [rng.choice([0, 1, 33, 1024, 8192, 16383, 16384, 248320, int(2 ** rng.uniform(0, 18))])
              for _ in range(2 if mode == hip.GemvMode.kSwiglu else rng.randint(1, 3))]
         if mode == hip.GemvMode.kSwiglu:
@@ -51,19 +51,19 @@ def test_every_choice_keeps_the_order_of_the_sums(cus):
 
 
 @pytest.mark.parametrize("cus", CUS)
-@pytest.mark.parametrize("K", [256, 1024, 2176, 5120])
+@pytest.mark.parametrize("K", [256, 1024, 3968, 4096, 5120])
 def test_tile_follows_tiles_per_cu(cus, K):
     """The lines lie at counts of 32 x 32 tiles per CU."""
     def at(tiles, M=32):  # so many tiles of one row group, over as many segments as keep N below 16384
         n = [tiles // 3 * 32, tiles // 3 * 32, (tiles - 2 * (tiles // 3)) * 32]
         return hip.gemm_tile(cus, n, K, M)
-    few, one, two, four = (1, 1, 8 if K > 2048 else 4), (1, 4, 1), (1, 2, 8), (1, 2, 4)
+    few, one, two, four = (1, 1, 8 if K >= 4096 else 4), (1, 4, 1), (1, 2, 8), (1, 2, 4)
     assert at(cus) == few and at(10 * cus + 1) == one
-    assert at(cus + 1) == (few if K <= 512 else two if K > 2048 else four)
+    assert at(cus + 1) == (few if K <= 512 else two if K >= 4096 else four)
     if K <= 512:
         assert at(4 * cus - 1) == few and at(4 * cus) == one
     elif cus < 256:  # (more tiles than 16384 outputs a segment have four shares)
-        assert at(2 * cus) == (two if K > 2048 else four) and at(2 * cus + 1) == four and at(10 * cus) == four
+        assert at(2 * cus) == (two if K >= 4096 else four) and at(2 * cus + 1) == four and at(10 * cus) == four
     assert at(16 * cus, 64) == (2, 4, 1) and at(16 * cus - 1, 64) == one
 
 

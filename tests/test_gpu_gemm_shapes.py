@@ -50,7 +50,7 @@ def wide(oracle, mat, sel, K, q, d, s):
 
 
 # (K, M, Ns, swiglu N): tiles of 32 x 32 outputs, by which the launch chooses. K has four
-# shares up to 2048, eight past that.
+# shares below 4096, eight from there.
 CASES = [
     (128, 17, [1, 33], 1),           # one activation tile with 15 dead rows, one block: three of four K groups have none
     (256, 32, [16070, 5], 8030),     # 504 / 502 tiles of few blocks: one wave x four groups, one full activation tile
@@ -63,13 +63,14 @@ CASES = [
     (4224, 64, [4200], 2200),        # 264 / 276 tiles: two waves x eight groups, 33 blocks
     (640, 65, [6917], 3500),         # 651 / 657 tiles: two waves x four groups; five blocks
     (640, 32, [16070, 5], 8030),     # the same of one full activation tile
-    (2176, 40, [16100, 20], 8100),   # 1008 / 1014 tiles: two waves x four groups of two shares, 17 blocks
+    (4224, 40, [16100, 20], 8100),   # 1008 / 1014 tiles: two waves x four groups of two shares
+    (2176, 40, [9000], 4500),        # 564 / 564 tiles: two waves x four groups of one share, 17 blocks
     (512, 520, [2000], 1000),        # 1071 / 1071 tiles of few blocks: four waves, K unsplit
     (1152, 1000, [3000], 1500),      # 3008 / 3008 tiles: four waves, K unsplit, four shares
-    (2176, 900, [3000], 1500),       # 2726 / 2726 tiles: the same, eight shares of two or three blocks
+    (4224, 900, [3000], 1500),       # 2726 / 2726 tiles: the same, eight shares of four or five blocks
     (256, 200, [18733], 9400),       # 4102 / 4116 tiles: four waves, K unsplit
     (256, 513, [15500], 7800),       # 8245 / 8296 tiles: 64 activation rows a wave, the last tile nearly empty
-    (2176, 513, [15500], 7800),      # the same, eight shares
+    (4224, 513, [15500], 7800),      # the same, eight shares
 ]
 
 
@@ -130,7 +131,7 @@ def test_t32_modes_and_edges(hip, oracle, K, M, Ns, N2):
 
 
 # one launch for each tile: (tile, K, M, N)
-DUMPS = [((1, 1, 4), 128, 17, 45), ((1, 1, 8), 2176, 40, 45), ((1, 2, 8), 2176, 64, 4200), ((1, 2, 4), 640, 40, 8205),
+DUMPS = [((1, 1, 4), 128, 17, 45), ((1, 1, 8), 4224, 40, 45), ((1, 2, 8), 4224, 64, 4200), ((1, 2, 4), 640, 40, 8205),
          ((1, 4, 1), 128, 513, 2005), ((2, 4, 1), 128, 513, 15500)]
 
 
@@ -217,7 +218,7 @@ def test_dot4_two_rows_equal_one_row_launches(hip, oracle, K, N):
     assert np.array_equal(I.cpu().numpy(), oracle.gemv_i32(mats[0][0], K, q, s))
 
 
-@pytest.mark.parametrize("K,wide_n", [(128, 9000), (640, 9000), (1152, 9000), (2176, 16390), (4224, 9000),
+@pytest.mark.parametrize("K,wide_n", [(128, 9000), (640, 9000), (1152, 9000), (4224, 16390), (4992, 9000),
                                       (12416, 9000)])
 def test_t32_rows_do_not_depend_on_the_launch(hip, K, wide_n):
     """More than 16 rows: an output's bits are the same however many rows and
